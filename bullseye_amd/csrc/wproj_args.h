@@ -29,6 +29,7 @@ struct WArgs {
     uint32_t M;                        // class width (odd)
     uint32_t lanes_per_stream, streams_per_block;
     float wmax_f;
+    double inv_wmax;                   // tiled gridder: 1 / wmax_f
     // Stream decomposition of the launch (read from the launch's own arguments, not a batched
     // facet's): rows per segment and segments per (baseline, channel block).  A launch whose
     // segments span several classification segments of base_rows rows walks only the rows of

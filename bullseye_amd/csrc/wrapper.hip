@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "host_common.h"
+#include "wtile.h"
 
 namespace bam {
 
@@ -77,7 +78,7 @@ struct State {
     DevBuf out_tmp, fft_scratch, fft_real, jinv, walk, dg_model, dg_out, stokes_tmp, dft_smp,
         dft_comp;
     // w-projection: taps re-laid per (plane, frac_v, frac_u), per-plane supports and sums
-    DevBuf wtaps_f, wtaps_d, wplane_off, wplane_half, wplane_norm, wcls, wlist;
+    DevBuf wtaps_f, wtaps_d, wplane_off, wplane_half, wplane_norm, wcls, wlist, wtile;
     DevBuf wctaps_f, wctaps_d, wcplane_off;   // column tables of the narrow classes
     std::vector<uint32_t> wplane_half_req;   // from bullseye_set_wplane_support
     std::vector<uint32_t> wplane_half_host;
@@ -499,6 +500,124 @@ static size_t aa_call_table_bytes(const gridding_parameters *p, int mode) {
     return n;
 }
 
+// W-projection by support classes (wproj.hip), for calls whose bins wtile_plan cannot number:
+// streams are segments of 32 rows of a baseline; the device classifies every (segment, channel
+// block) by its support class and sorts them by class, and one persistent launch per class width
+// takes its list from there (no host round trip).
+static int grid_classes(GridArgs a, size_t rows, size_t B, float wmax_f, const void *taps,
+                        int mode) {
+    const WListPlan lp = wproj_list_plan((uint32_t)rows, (uint32_t)B, a.n_chan_blocks);
+    if (lp.entries >= 0x7fffffffull || lp.entries * g.F > 0xffffffffull)
+        return fail("too many w-projection streams");
+    a.n_segments = 0;   // streams come from the device lists
+    a.n_streams = lp.entries * g.F;
+    void *lws = nullptr;
+    HIP_TRY(table(g.wlist, lp.total, &lws));
+    HIP_TRY(wproj_build_lists(a, lp, lws, g.wplane_half.as<uint32_t>(), (uint32_t)g.wplanes,
+                              wmax_f, g.stream));
+    const void *ctaps = g.path == PATH_FP64 ? g.wctaps_d.p : g.wctaps_f.p;
+    uint32_t max_m = 1;
+    for (uint32_t h : g.wplane_half_host) max_m = std::max(max_m, 2 * h + 1);
+    // one persistent launch per class width, dealt over the stream and the side streams so
+    // that a launch's tail and the small classes overlap other classes' work
+    HIP_TRY(hipEventRecord(g.wfork, g.stream));
+    for (int i = 0; i < State::WSIDE; ++i) HIP_TRY(hipStreamWaitEvent(g.wside[i], g.wfork, 0));
+    // Classes wider than 31 hold few samples each: one launch per lane shape (two or four
+    // residue pairs per lane) walks all of them, each stream at its own width, instead of
+    // one latency-bound launch per class.  They go first, so that their long streams overlap
+    // the wide-parallel launches of the narrower classes, which follow widest first.
+    std::vector<std::pair<uint32_t, uint32_t>> order;
+    if (max_m > 45) order.push_back({47, max_m});
+    if (max_m > 31) order.push_back({33, std::min<uint32_t>(max_m, 45)});
+    for (int M = (int)std::min<uint32_t>(max_m, 31); M >= 1; M -= 2)
+        order.push_back({(uint32_t)M, (uint32_t)M});
+    hipError_t le = hipSuccess;
+    for (size_t i = 0; i < order.size() && le == hipSuccess; ++i) {
+        const int turn = (int)(i % (State::WSIDE + 1));
+        le = launch_wproj_device_list(a, lp, lws, taps, g.wplane_off.as<uint64_t>(), ctaps,
+                                      g.wcplane_off.as<uint64_t>(),
+                                      g.wplane_half.as<uint32_t>(),
+                                      g.wplane_norm.as<double>(), (uint32_t)g.wplanes,
+                                      g.w_nf, g.w_fbase, order[i].first, order[i].second,
+                                      wmax_f, mode, g.path,
+                                      turn ? g.wside[turn - 1] : g.stream);
+    }
+    // joined also after a failed launch: later work on the stream (the next call's class
+    // lists) must not overtake what was launched
+    for (int i = 0; i < State::WSIDE; ++i) {
+        HIP_TRY(hipEventRecord(g.wjoin[i], g.wside[i]));
+        HIP_TRY(hipStreamWaitEvent(g.stream, g.wjoin[i], 0));
+    }
+    HIP_TRY(le);
+    return 0;
+}
+
+// W-projection through on-chip tiles (wtile.hip), in passes over facets (and rows, where one
+// facet's samples are too many) whose records fit the workspace.  tiled: whether it applied.
+static int grid_tiles(const GridArgs &a, size_t rows, float wmax_f, const void *taps, int mode,
+                      bool &tiled) {
+    tiled = !(g.opts.reserved[0] & 2);
+    if (!tiled || !rows || !a.chan) return 0;
+    const bool fp64 = g.path == PATH_FP64;
+    const int nc = mode == MODE_2 ? 2 : (mode == MODE_4 || mode == MODE_4J) ? 4 : 1;
+    uint8_t widths[32] = {};
+    uint32_t lo = 31, hi = 0;
+    for (uint32_t h : g.wplane_half_host) {
+        widths[h] = 1;
+        lo = std::min(lo, h);
+        hi = std::max(hi, h);
+    }
+    const uint64_t spots1 = (uint64_t)a.cube * wt::tiles_of(a.nx) * wt::tiles_of(a.ny);
+    const size_t rec = sizeof(wt::Head) + 4 + (size_t)nc * (fp64 ? 16 : 8);
+    // 4 GiB of records, halved while the workspace cannot be had
+    for (uint64_t cap = g.opts.reserved[1] ? g.opts.reserved[1] : ((size_t)4 << 30) / rec;;
+         cap /= 2) {
+        const uint64_t rows1 = std::min<uint64_t>(rows, std::max<uint64_t>(1, cap / a.chan));
+        uint64_t F1 = std::max<uint64_t>(1, cap / (rows * a.chan));
+        F1 = std::min<uint64_t>(std::min<uint64_t>(F1, a.facets), 65535);
+        wt::Plan pl;
+        while (F1 > 1 && !wtile_plan(pl, rows1 * a.chan * F1, spots1 * F1, lo, hi, nc, fp64))
+            F1 = (F1 + 1) / 2;
+        if (!wtile_plan(pl, rows1 * a.chan * F1, spots1 * F1, lo, hi, nc, fp64)) {
+            tiled = false;
+            return 0;
+        }
+        const hipError_t e = g.wtile.ensure(pl.total);
+        if (e == hipErrorOutOfMemory && cap > (1u << 20)) {
+            (void)hipGetLastError();
+            continue;
+        }
+        HIP_TRY(e);
+        wt::TArgs t{};
+        t.w.g = a;
+        t.w.taps = taps;
+        t.w.plane_off = g.wplane_off.as<uint64_t>();
+        t.w.plane_half = g.wplane_half.as<uint32_t>();
+        t.w.plane_norm = g.wplane_norm.as<double>();
+        t.w.wplanes = (uint32_t)g.wplanes;
+        t.w.nf = g.w_nf;
+        t.w.fbase = g.w_fbase;
+        t.w.wmax_f = wmax_f;
+        t.w.inv_wmax = 1.0 / (double)wmax_f;
+        for (uint64_t f0 = 0; f0 < a.facets; f0 += F1)
+            for (uint64_t r0 = 0; r0 < rows; r0 += rows1) {
+                t.f0 = (uint32_t)f0;
+                t.nfacets = (uint32_t)std::min<uint64_t>(F1, a.facets - f0);
+                t.row0 = (uint32_t)r0;
+                t.row1 = (uint32_t)std::min<uint64_t>(rows, r0 + rows1);
+                // the last pass may hold fewer facets or rows: its bins are planned for itself
+                wt::Plan one;
+                if (!wtile_plan(one, (uint64_t)(t.row1 - t.row0) * a.chan * t.nfacets,
+                                spots1 * t.nfacets, lo, hi, nc, fp64))
+                    return fail("w-projection workspace plan");
+                HIP_TRY(g.wtile.ensure(one.total));
+                HIP_TRY(wtile_grid(t, one, g.wtile.p, mode, fp64, widths, g.stream, g.wside,
+                                   State::WSIDE, g.wfork, g.wjoin));
+            }
+        return 0;
+    }
+}
+
 // One gridding call.  noalloc (bullseye_grid_noalloc): the tables come from the scratch arena
 // and no timing events are created, so the call allocates nothing.
 static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
@@ -597,59 +716,16 @@ static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
     }
 
     if (wproj) {
-        // w-projection: streams are segments of 32 rows of a baseline; the device classifies
-        // every (segment, channel block) by its support class and sorts them by class, and
-        // one persistent launch per class width takes its list from there (no host round trip)
         const float wmax_f = (float)p->wmax_est;
         if (!(wmax_f > 0)) return fail("wmax_est must be > 0 for w-projection");
-        const WListPlan lp = wproj_list_plan((uint32_t)rows, (uint32_t)B, a.n_chan_blocks);
-        if (lp.entries >= 0x7fffffffull || lp.entries * g.F > 0xffffffffull)
-            return fail("too many w-projection streams");
-        a.n_segments = 0;   // streams come from the device lists
-        a.n_streams = lp.entries * g.F;
-        void *lws = nullptr;
-        HIP_TRY(table(g.wlist, lp.total, &lws));
-        HIP_TRY(wproj_build_lists(a, lp, lws, g.wplane_half.as<uint32_t>(), (uint32_t)g.wplanes,
-                                  wmax_f, g.stream));
         const void *taps = g.path == PATH_FP64 ? g.wtaps_d.p : g.wtaps_f.p;
-        const void *ctaps = g.path == PATH_FP64 ? g.wctaps_d.p : g.wctaps_f.p;
-        uint32_t max_m = 1;
-        for (uint32_t h : g.wplane_half_host) max_m = std::max(max_m, 2 * h + 1);
         HIP_TRY(hipEventRecord(tc.k0, g.stream));
-        // one persistent launch per class width, dealt over the stream and the side streams so
-        // that a launch's tail and the small classes overlap other classes' work
-        HIP_TRY(hipEventRecord(g.wfork, g.stream));
-        for (int i = 0; i < State::WSIDE; ++i) HIP_TRY(hipStreamWaitEvent(g.wside[i], g.wfork, 0));
-        // Classes wider than 31 hold few samples each: one launch per lane shape (two or four
-        // residue pairs per lane) walks all of them, each stream at its own width, instead of
-        // one latency-bound launch per class.  They go first, so that their long streams overlap
-        // the wide-parallel launches of the narrower classes, which follow widest first.
-        std::vector<std::pair<uint32_t, uint32_t>> order;
-        if (max_m > 45) order.push_back({47, max_m});
-        if (max_m > 31) order.push_back({33, std::min<uint32_t>(max_m, 45)});
-        for (int M = (int)std::min<uint32_t>(max_m, 31); M >= 1; M -= 2)
-            order.push_back({(uint32_t)M, (uint32_t)M});
-        hipError_t le = hipSuccess;
-        for (size_t i = 0; i < order.size() && le == hipSuccess; ++i) {
-            const int turn = (int)(i % (State::WSIDE + 1));
-            le = launch_wproj_device_list(a, lp, lws, taps, g.wplane_off.as<uint64_t>(), ctaps,
-                                          g.wcplane_off.as<uint64_t>(),
-                                          g.wplane_half.as<uint32_t>(),
-                                          g.wplane_norm.as<double>(), (uint32_t)g.wplanes,
-                                          g.w_nf, g.w_fbase, order[i].first, order[i].second,
-                                          wmax_f, mode, g.path,
-                                          turn ? g.wside[turn - 1] : g.stream);
-        }
-        // joined also after a failed launch: later work on the stream (the next call's class
-        // lists) must not overtake what was launched
-        for (int i = 0; i < State::WSIDE; ++i) {
-            HIP_TRY(hipEventRecord(g.wjoin[i], g.wside[i]));
-            HIP_TRY(hipStreamWaitEvent(g.stream, g.wjoin[i], 0));
-        }
-        HIP_TRY(le);
+        bool tiled = false;
+        if (grid_tiles(a, rows, wmax_f, taps, mode, tiled)) return 1;
+        if (!tiled && grid_classes(a, rows, B, wmax_f, taps, mode)) return 1;
     } else {
         const bool specialised = romein_w_groups_per_wave(W, mode, g.path) > 0 &&
-                                 !g.opts.reserved[0];
+                                 !(g.opts.reserved[0] & 1);
         if (specialised) {
             const bool four = mode == MODE_4 || mode == MODE_4J;
             a.pol_contig = (four && !psf && p->number_of_polarization_terms == 4 &&
@@ -877,7 +953,7 @@ static void release_resources() {
                       &g.rowrec, &g.chanrec,
                       &g.counts, &g.ws, &g.out_tmp,
                       &g.fft_scratch, &g.fft_real, &g.jinv, &g.wtaps_f, &g.wtaps_d,
-                      &g.wplane_off, &g.wplane_half, &g.wplane_norm, &g.wcls, &g.wlist, &g.walk,
+                      &g.wplane_off, &g.wplane_half, &g.wplane_norm, &g.wcls, &g.wlist, &g.wtile, &g.walk,
                       &g.wctaps_f, &g.wctaps_d, &g.wcplane_off,
                       &g.dg_model, &g.dg_out, &g.stokes_tmp, &g.dft_smp, &g.dft_comp};
     for (DevBuf *b : bufs) b->release();

@@ -205,7 +205,9 @@ typedef struct bullseye_options {
     uint32_t walk_order;        /* order of a stream's samples: 0 = whichever moves the kernel
                                    footprint less per step, measured from the data; 1 =
                                    channels inner; 2 = time inner */
-    uint32_t reserved[9];       /* reserved[0] = 1 forces the generic (any-support) kernel */
+    uint32_t reserved[9];       /* reserved[0]: bit 0 forces the generic (any-support) AA
+                                   kernel, bit 1 the w-projection class kernels; reserved[1]:
+                                   w-projection records per pass (0 = up to 4 GiB of them) */
 } bullseye_options;
 
 int bullseye_set_options(const bullseye_options *options);
