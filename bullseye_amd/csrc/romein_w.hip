@@ -108,36 +108,39 @@ template <int MODE, int PATH, int W> struct GridderW {
         }
     }
 
+    // x mod W, for x < 2^22 by a float reciprocal (x + 1/2 lies at least 1/2 from a multiple of
+    // W, the rounding below 2^-23 x); the integer division's two 32-bit products take a quarter
+    // of the rate each.
+    static __device__ __forceinline__ int residue(int x, bool small) {
+        if (!small) return x % W;
+        const int q = (int)fmaf((float)x, 1.0f / W, 0.5f / W);
+        return x - (int)__umul24((uint32_t)q, W);
+    }
+
     // Prepare sample (sorted row ri, channel c); returns false when it contributes nothing.
     // The checks and their order (and so the errors raised) are those of a gather straight from
     // the row arrays: spw range, enabled channel, grid slice range, row flag and field, then the
-    // Jones ids.
+    // Jones ids; they are told apart only for a sample that fails one.
+    // wt: the weights, ts: the tap sum of the sample's footprint (normalisation terms wt * ts).
     static __device__ __forceinline__ bool prep(const GridArgs &a, const FacetGeom *__restrict__ gp,
                                                 const T *stap, const double *sts,
                                                 const ChanRec *schan, uint32_t ri,
                                                 uint64_t jfacet, uint32_t c, R_t &r,
-                                                double nw[NC]) {
+                                                T (&wt)[NC], double &ts) {
         const RowRec rr = load_row_record(a.rowrec + ri);
         const uint32_t s = rr.spw;
-        if (s >= a.spw_count) {
-            atomicOr(a.error_flag, 4);
-            return false;
-        }
-        const uint32_t fc = s * a.chan + c;
-        const ChanRec ch = schan[fc];   // the channel table is staged in LDS
-        if (!ch.enabled) return false;
-        if (ch.cgi >= a.cube) {
-            atomicOr(a.error_flag, 4);
-            return false;
-        }
-        if (!(rr.state & ROW_USABLE)) return false;
-        if constexpr (MODE == MODE_4J) {
-            // raised here, before the visibility loads, so that the Jones loads issue with them
-            // (nothing between this point and the Jones correction can drop the sample)
-            if (rr.state & ROW_BAD_IDS) {
+        // the channel table is staged in LDS, so spw_count * chan <= CHAN_LDS_MAX
+        const bool in_table = s < a.spw_count;
+        const uint32_t fc = in_table ? __umul24(s, a.chan) + c : 0u;
+        const ChanRec ch = schan[fc];
+        const uint32_t want = MODE == MODE_4J ? (ROW_USABLE | ROW_BAD_IDS) : ROW_USABLE;
+        if (!in_table || !ch.enabled || ch.cgi >= a.cube || (rr.state & want) != ROW_USABLE) {
+            // BAD_IDS is raised here, before the visibility loads, so that the Jones loads issue
+            // with them (nothing between this point and the Jones correction drops the sample)
+            if (!in_table || (ch.enabled && (ch.cgi >= a.cube ||
+                                             ((rr.state & ROW_USABLE) && MODE == MODE_4J))))
                 atomicOr(a.error_flag, 4);
-                return false;
-            }
+            return false;
         }
         const uint32_t row = rr.row;
         const double rw = ch.rw;
@@ -155,12 +158,11 @@ template <int MODE, int PATH, int W> struct GridderW {
             }
         }
         cpx<T> vis[NC];
-        T wt[NC];
         if constexpr (MODE == MODE_PSF) {
             vis[0] = {T(1), T(0)};
             wt[0] = T(1);
         } else {
-            const size_t base = ((size_t)row * a.chan + c) * a.npol;
+            const size_t base = (size_t)row * (a.chan * a.npol) + c * a.npol;
             if constexpr (NC == 4) {
                 if (a.pol_contig) {
                     visibility_base_type vv[8];
@@ -214,7 +216,7 @@ template <int MODE, int PATH, int W> struct GridderW {
                 cs = c_;
             } else {
                 float s_, c_;
-                sincospif((float)fr, &s_, &c_);
+                sincospi_unit((float)fr, &s_, &c_);
                 sn = s_;
                 cs = c_;
             }
@@ -240,8 +242,9 @@ template <int MODE, int PATH, int W> struct GridderW {
 #pragma unroll
         for (int k = 0; k < NC; ++k) r.vis[k] = vis[k];
         // residue-ordered tap runs: tap j of a run is conv[f + ((j - m) mod W) * OS]
-        const int tu = fu * (2 * W) + W - x0 % W;
-        const int tv = fv * (2 * W) + W - y0 % W;
+        const bool small = (a.nx | a.ny) < (1u << 22);
+        const int tu = (int)__umul24((uint32_t)fu, 2 * W) + W - residue(x0, small);
+        const int tv = (int)__umul24((uint32_t)fv, 2 * W) + W - residue(y0, small);
         if constexpr (TR) {
 #pragma unroll
             for (int j = 0; j < W; ++j) {
@@ -252,9 +255,7 @@ template <int MODE, int PATH, int W> struct GridderW {
             r.tu = tu;
             r.tv = tv;
         }
-        const double ts = sts[fu] * sts[fv];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) nw[k] = (double)wt[k] * ts;
+        ts = sts[fu] * sts[fv];
         return true;
     }
 
@@ -487,8 +488,9 @@ template <int MODE, int PATH, int W> struct GridderW {
                     const uint32_t i = (so & 1) ? inner - 1 - si : si;
                     const uint32_t tr = tin ? i : so, j = tin ? so : i;
                     const uint32_t c = c_lo + j;
-                    double nw[NC];
-                    if (prep(a, gp, stap, sts, schan, b0 + r_lo + tr, jfacet, c, rec, nw)) {
+                    T wt[NC];
+                    double ts;
+                    if (prep(a, gp, stap, sts, schan, b0 + r_lo + tr, jfacet, c, rec, wt, ts)) {
                         ++cnt;
                         if constexpr (MODE != MODE_PSF) {
                             if (rec.cgi != ncgi) {
@@ -496,7 +498,7 @@ template <int MODE, int PATH, int W> struct GridderW {
                                 ncgi = rec.cgi;
                             }
 #pragma unroll
-                            for (int k = 0; k < NC; ++k) nacc[k] += nw[k];
+                            for (int k = 0; k < NC; ++k) nacc[k] = fma((double)wt[k], ts, nacc[k]);
                         }
                     } else {
                         rec.cgi = -1;
@@ -636,8 +638,278 @@ template <int MODE, int PATH, int W> struct GridderW {
     }
 };
 
+// ---------- 4 correlations on the FP32 paths, W = 7: one stream per wavefront, matrix cores ------
+// The run update of a sample is the outer product of its 7 v taps with the 56 values
+// vis[corr][re, im] * u tap.  v_mfma_f32_4x4x1_16b multiplies one broadcast block of 4 A values
+// with 64 B values, one per lane: two of them are the 8 (7) x 64 (56) product, and their
+// accumulator layout (a lane's column, 4 rows a register quad) is Romein's ownership: lane
+// 8 a + q owns u-residue a of value q = 2 corr + (re, im), its registers the 7 v-residues.  A
+// product is one FMA, rounded as fmaf rounds it (checked bit for bit, denormals included), so
+// the sums are those of the FMA chains of GridderW.  The 8 lanes beyond the 56 columns carry the
+// v taps: one register is both operands.
+//
+// Per sample and wavefront: one multiply, two MFMAs (10.3 cycles each, measured) and half an LDS
+// instruction (128-bit reads of four samples), against 16 FMAs and multiplies and the record
+// reads for two samples in GridderW.  The two pipes do not overlap here (an MFMA and four FMAs
+// take 25.4 cycles, 10.3 + 15.1), so what bounds the kernel is their sum: at 25 facets x 4
+// correlations with Jones terms (774 M samples) 35.1 -> 21.5 ms, 8.6 vector instructions and 2
+// MFMAs a sample against 19.6.  64 samples are prepared by 64 lanes (56 there), the run
+// boundaries are one ballot and the control is scalar.  A cell's 4 correlations are 64
+// consecutive bytes of the grid in 8 adjacent lanes: one request a flushed cell instead of two.
+template <int MODE, int PATH> struct Wave4 {
+    static constexpr int W = 7, NC = 4, COLS = 8 * W;
+    typedef GridderW<MODE, PATH, W> Prep;
+    typedef typename Prep::R_t R_t;
+    static constexpr bool KAHAN = PathTraits<PATH>::KAHAN;
+    // LDS of a wavefront: rows of 64 samples (+ 4 floats, so that the 16 rows an instruction
+    // reads start on different banks): vis 0-7, u taps 8-14, v taps 15-21, ones 22
+    static constexpr int ROW = 68, NROW = 23;
+    static constexpr int WAVE_BYTES = NROW * ROW * 4;
+    // samples a run holds at most: against 64 bits, the grids of three workloads are 2 to 9 %
+    // closer than with GridderW's runs of up to 28 (32: 2 to 10 % further off)
+    static constexpr int RUN = 24;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+
+    // The lane's 7 sums.  Compensated: the true sum is s + n, and a run continues n (minus the
+    // Kahan correction), so opening one costs nothing; uncompensated: n is the sum.
+    struct Sums {
+        float s[W];
+        f4 n0, n1;
+        __device__ __forceinline__ float n(int r) const { return r < 4 ? n0[r] : n1[r - 4]; }
+        __device__ __forceinline__ void set_n(int r, float v) {
+            if (r < 4)
+                n0[r] = v;
+            else
+                n1[r - 4] = v;
+        }
+        __device__ __forceinline__ void zero(int r) {
+            s[r] = 0.0f;
+            set_n(r, 0.0f);
+        }
+        __device__ __forceinline__ double value(int r) const {
+            return KAHAN ? (double)s[r] + (double)n(r) : (double)n(r);
+        }
+        // one Kahan step ends a run
+        __device__ __forceinline__ void close() {
+            if constexpr (KAHAN) {
+#pragma unroll
+                for (int r = 0; r < W; ++r) {
+                    const float y = n(r), t = s[r] + y;
+                    set_n(r, y - (t - s[r]));
+                    s[r] = t;
+                }
+            }
+        }
+    };
+
+    // One sample: x is the lane's column value (lanes below 56) or v tap (the others).
+    static __device__ __forceinline__ void add(float x, Sums &s) {
+        s.n0 = __builtin_amdgcn_mfma_f32_4x4x1f32(x, x, s.n0, 4, 14, 0);
+        s.n1 = __builtin_amdgcn_mfma_f32_4x4x1f32(x, x, s.n1, 4, 15, 0);
+    }
+
+    static __device__ __forceinline__ int mod_w(int v) {  // v in (-W, 2W)
+        v = v < 0 ? v + W : v;
+        return v >= W ? v - W : v;
+    }
+
+    // Flush row r of the lanes in `who` (bit per lane) at grid row `row`.
+    static __device__ __forceinline__ void flush(double *cell, bool who, Sums &s, int r) {
+        if (!who) return;
+        const double x = s.value(r);
+        if (x != 0.0) unsafeAtomicAdd(cell, x);
+        s.zero(r);
+    }
+
+    // Footprint (scalar) the sums belong to, and its move to (x0, y0, cgi).
+    struct Own {
+        int x0, y0, cgi;
+    };
+    static __device__ __forceinline__ double *column(const GridArgs &a, uint32_t facet, int cgi,
+                                                     int x, int q) {
+        return a.grid + ((((size_t)facet * a.cube + cgi) * a.ny * a.nx + x) * (size_t)a.pstride) * 2 + q;
+    }
+    static __device__ __forceinline__ void move(const GridArgs &a, uint32_t facet, int lane, Own &o,
+                                                int x0, int y0, int cgi, Sums &s) {
+        if (o.cgi >= 0) {
+            const int xo = o.x0 + mod_w((lane >> 3) - o.x0 % W);
+            const bool mine = lane < COLS;
+            const bool col = mine && ((unsigned)(xo - x0) >= (unsigned)W);
+            const int pym = o.y0 % W;
+            double *base = column(a, facet, o.cgi, xo, lane & 7);
+            const size_t rs = (size_t)a.nx * a.pstride * 2u;
+#pragma unroll
+            for (int r = 0; r < W; ++r) {
+                const int yo = o.y0 + mod_w(r - pym);
+                const bool row = cgi != o.cgi || (unsigned)(yo - y0) >= (unsigned)W;
+                flush(base + (size_t)yo * rs, row ? mine : col, s, r);
+            }
+        }
+        o.x0 = x0;
+        o.y0 = y0;
+        o.cgi = cgi;
+    }
+
+    static __device__ __forceinline__ int scalar(int v, int l) {
+        return __builtin_amdgcn_readlane(v, l);
+    }
+
+    static __device__ void run(const GridArgs &a, const float *stap, const double *sts,
+                               const ChanRec *schan, float *lds) {
+        int nkey = -1;
+        double nacc[NC] = {0, 0, 0, 0};
+        unsigned long long cnt = 0;
+        walk(a, stap, sts, schan, lds, nkey, nacc, cnt);
+        publish_norm<NC>(a, nkey, nacc);
+        publish_counts(a, cnt, cnt * (unsigned long long)(W * W));
+    }
+
+    static __device__ __forceinline__ void walk(const GridArgs &a, const float *stap,
+                                                const double *sts, const ChanRec *schan, float *lds,
+                                                int &nkey, double (&nacc)[NC],
+                                                unsigned long long &cnt) {
+        const int lane = threadIdx.x & 63;
+        const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const uint64_t stream = (uint64_t)xcd_block() * (BLOCK / 64) + wave;
+        if (stream >= a.n_streams) return;
+        uint64_t t = stream;
+        const uint32_t facet = (uint32_t)(t % a.facets);
+        t /= a.facets;
+        const uint32_t seg = (uint32_t)(t % a.n_segments);
+        t /= a.n_segments;
+        const uint32_t cb = (uint32_t)(t % a.n_chan_blocks);
+        const uint32_t bl = (uint32_t)(t / a.n_chan_blocks);
+        const uint32_t b0 = a.bl_start[bl];
+        const uint32_t nb = a.bl_start[bl + 1] - b0;
+        const uint32_t r_lo = (uint32_t)(((uint64_t)nb * seg) / a.n_segments);
+        const uint32_t r_hi = (uint32_t)(((uint64_t)nb * (seg + 1)) / a.n_segments);
+        const uint32_t c_lo = cb * a.chan_per_stream;
+        const uint32_t ncb = min(a.chan, c_lo + a.chan_per_stream) - c_lo;
+        const uint32_t nrows = r_hi - r_lo;
+        const uint32_t nsamp = nrows * ncb;
+        const bool tin = *a.time_inner != 0;
+        const FacetGeom *gp = a.geom + facet;
+        const uint64_t jfacet = (uint64_t)facet * a.spw_count * a.chan;
+
+        // the lane's two operand rows: value q and u tap a, or a v tap and one
+        const bool tap_lane = lane >= COLS;
+        const f4 *row_a = reinterpret_cast<const f4 *>(
+            lds + (tap_lane ? min(15 + lane - COLS, 21) : lane & 7) * ROW);
+        const f4 *row_b = reinterpret_cast<const f4 *>(lds + (tap_lane ? 22 : 8 + (lane >> 3)) * ROW);
+        lds[22 * ROW + lane] = 1.0f;
+
+        Sums s;
+#pragma unroll
+        for (int r = 0; r < W; ++r) s.zero(r);
+        s.n1[3] = 0.0f;
+        Own own = {-1, -1, -1};
+        int ncgi = -1;
+        const uint32_t inner = max(1u, tin ? nrows : ncb);
+        uint32_t so = (uint32_t)lane / inner, si = (uint32_t)lane - so * inner;
+        const uint32_t dso = 64u / inner, dsi = 64u - dso * inner;
+        for (uint32_t step0 = 0; step0 < nsamp; step0 += 64) {
+            // issue priority: low while preparing (mostly waiting on loads), high while walking
+            __builtin_amdgcn_s_setprio(0);
+            R_t rec;
+            rec.cgi = -1;
+            rec.x0 = rec.y0 = 0;
+            if (step0 + lane < nsamp) {
+                const uint32_t i = (so & 1) ? inner - 1 - si : si;
+                const uint32_t tr = tin ? i : so, j = tin ? so : i;
+                float wt[NC];
+                double ts;
+                if (Prep::prep(a, gp, stap, sts, schan, b0 + r_lo + tr, jfacet, c_lo + j, rec, wt,
+                               ts)) {
+                    ++cnt;
+                    if (rec.cgi != ncgi) {
+                        if (ncgi >= 0) flush_norm_lane<NC>(a, (int)(facet * a.cube + ncgi), nacc);
+                        ncgi = rec.cgi;
+                    }
+#pragma unroll
+                    for (int k = 0; k < NC; ++k) nacc[k] = fma((double)wt[k], ts, nacc[k]);
+                } else {
+                    rec.cgi = -1;
+                }
+            }
+            si += dsi;
+            so += dso;
+            if (si >= inner) {
+                si -= inner;
+                ++so;
+            }
+            const uint64_t valid = __ballot(rec.cgi >= 0);
+            if (!valid) continue;
+            if (rec.cgi < 0) {   // contributes nothing, on whatever footprint is open
+#pragma unroll
+                for (int k = 0; k < NC; ++k) rec.vis[k] = {0.0f, 0.0f};
+#pragma unroll
+                for (int j = 0; j < W; ++j) rec.cu[j] = rec.cv[j] = 0.0f;
+            }
+            // a valid sample on another footprint than the valid one before it opens a run
+            const uint64_t below = valid & ((1ull << lane) - 1);
+            const int prev = below ? 63 - __clzll((long long)below) : lane;
+            const int qx = __shfl(rec.x0, prev, 64), qy = __shfl(rec.y0, prev, 64);
+            const int qc = __shfl(rec.cgi, prev, 64);
+            const bool moved = below ? (qx != rec.x0 || qy != rec.y0 || qc != rec.cgi)
+                                     : (rec.x0 != own.x0 || rec.y0 != own.y0 || rec.cgi != own.cgi);
+            const uint64_t opens = __ballot(rec.cgi >= 0 && moved);
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                lds[(2 * k) * ROW + lane] = rec.vis[k].re;
+                lds[(2 * k + 1) * ROW + lane] = rec.vis[k].im;
+            }
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                lds[(8 + j) * ROW + lane] = rec.cu[j];
+                lds[(15 + j) * ROW + lane] = rec.cv[j];
+            }
+            __builtin_amdgcn_s_setprio(3);
+            wave_sync();
+            // the step in spans of one run each: up to the next sample that opens a run, at most
+            // RUN samples.  Samples are read and multiplied in aligned quads, those outside
+            // the span with zero (a run boundary costs one more quad).
+            const int n = (int)min(64u, nsamp - step0);
+            int pos = 0;
+            do {
+                if ((opens >> pos) & 1)
+                    move(a, facet, lane, own, scalar(rec.x0, pos), scalar(rec.y0, pos),
+                         scalar(rec.cgi, pos), s);
+                const uint64_t later = opens & ~((2ull << pos) - 1);
+                int end = later ? __ffsll((unsigned long long)later) - 1 : n;
+                end = min(end, (pos + RUN) & ~3);
+                const int q1 = (end + 3) >> 2;
+                int q = pos >> 2;
+                f4 xa = row_a[q], xb = row_b[q];
+                for (; q < q1; ++q) {
+                    f4 x = xa * xb;
+                    xa = row_a[q + 1];   // the next quad's (or padding), read while this one is added
+                    xb = row_b[q + 1];
+                    if (4 * q < pos || 4 * q + 4 > end) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            x[k] = (4 * q + k >= pos && 4 * q + k < end) ? x[k] : 0.0f;
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) add(x[k], s);
+                }
+                s.close();
+                pos = end;
+            } while (pos < n);
+            wave_sync();
+        }
+        if (own.cgi >= 0) move(a, facet, lane, own, own.x0, own.y0, -1, s);
+        nkey = ncgi >= 0 ? (int)(facet * a.cube + ncgi) : -1;
+    }
+};
+
+// Whether streams of (mode, path, width) are walked one per wavefront (Wave4).
+constexpr bool one_per_wave(int mode, int path, int W) {
+    return W == 7 && path != PATH_FP64 && (mode == MODE_4 || mode == MODE_4J);
+}
+
 template <int MODE, int PATH, int W>
-__global__ __launch_bounds__(BLOCK) void romein_w_kernel(GridArgs a) {
+__global__ __launch_bounds__(BLOCK, one_per_wave(MODE, PATH, W) ? 4 : 1)
+void romein_w_kernel(GridArgs a) {
     typedef GridderW<MODE, PATH, W> Gd;
     typedef typename Gd::T T;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -658,20 +930,29 @@ __global__ __launch_bounds__(BLOCK) void romein_w_kernel(GridArgs a) {
     const uint32_t nfc = a.spw_count * a.chan;   // <= CHAN_LDS_MAX (launch_romein_w checks)
     for (uint32_t i = threadIdx.x; i < nfc; i += BLOCK) schan[i] = a.chanrec[i];
     __syncthreads();
-    Gd::run(a, stap, sts, schan,
-            smem + conv_bytes + ts_bytes + ((nfc * sizeof(ChanRec) + 15) & ~15u) +
-                (threadIdx.x >> 6) * Gd::WAVE_BYTES);
+    unsigned char *own = smem + conv_bytes + ts_bytes + ((nfc * sizeof(ChanRec) + 15) & ~15u);
+    if constexpr (one_per_wave(MODE, PATH, W)) {
+        typedef Wave4<MODE, PATH> W4;
+        W4::run(a, stap, sts, schan,
+                reinterpret_cast<float *>(own + (threadIdx.x >> 6) * W4::WAVE_BYTES));
+    } else {
+        Gd::run(a, stap, sts, schan, own + (threadIdx.x >> 6) * Gd::WAVE_BYTES);
+    }
 }
 
 template <int MODE, int PATH, int W> static hipError_t launch_t(const GridArgs &a, hipStream_t st) {
     typedef GridderW<MODE, PATH, W> Gd;
-    const uint64_t waves = (a.n_streams + Gd::GPW - 1) / Gd::GPW;
+    constexpr bool one = one_per_wave(MODE, PATH, W);
+    constexpr int gpw = one ? 1 : Gd::GPW;
+    const uint64_t waves = (a.n_streams + gpw - 1) / gpw;
     const uint64_t blocks = (waves + BLOCK / 64 - 1) / (BLOCK / 64);
     if (blocks == 0) return hipSuccess;
+    size_t wave_bytes = Gd::WAVE_BYTES;
+    if constexpr (one) wave_bytes = Wave4<MODE, PATH>::WAVE_BYTES;
     const size_t smem = ((rot_table_len(a.OS, W) * sizeof(typename Gd::T) + 15) & ~15u) +
                         (((a.OS + 1) * 8 + 15) & ~15u) +
                         (((size_t)a.spw_count * a.chan * sizeof(ChanRec) + 15) & ~(size_t)15) +
-                        (BLOCK / 64) * (size_t)Gd::WAVE_BYTES;
+                        (BLOCK / 64) * wave_bytes;
     if (!a.rowrec || !a.chanrec) return hipErrorInvalidValue;
     romein_w_kernel<MODE, PATH, W><<<dim3((uint32_t)blocks), dim3(BLOCK), smem, st>>>(a);
     return hipGetLastError();
@@ -703,6 +984,7 @@ hipError_t launch_romein_aa(const GridArgs &a, int mode, int path, hipStream_t s
 
 // Lane groups per wavefront for a support width, or 0 when no specialisation exists.
 int romein_w_groups_per_wave(int W, int mode, int path) {
+    if (rw::one_per_wave(mode, path, W)) return 1;
     const int split = (mode == MODE_4 || mode == MODE_4J) ? (path == PATH_FP64 ? 2 : 4) : 1;
     switch (W) {
         case 3: case 5: case 7: case 9: case 11: return 64 / (W * split);
