@@ -9,7 +9,7 @@
 // image-plane response of the sampled AA kernel (no counterpart in the reference).
 #include <hipfft/hipfft.h>
 
-#include "device_common.h"
+#include "host_common.h"
 
 namespace bam {
 
@@ -17,11 +17,12 @@ typedef visibility_base_type vis_t;
 
 // internal FP64 accumulation grid [F][C][ny][nx][pstride][2] <-> ABI grid
 // complex<grid_base_type>[F][C][P][ny][nx]
+// (err: nothing is written while the device error flag is set)
 __global__ void k_grid_to_abi(const double *g, grid_base_type *out, uint64_t slices_fc, uint32_t P,
-                              uint32_t pstride, uint64_t npix) {
+                              uint32_t pstride, uint64_t npix, const int *err) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t total = slices_fc * npix;
-    if (i >= total) return;
+    if (i >= total || (err && *err)) return;
     const uint64_t fc = i / npix, pix = i - fc * npix;
     const double *src = g + (fc * npix + pix) * pstride * 2;
     for (uint32_t p = 0; p < P; ++p) {
@@ -101,9 +102,14 @@ __global__ void k_ifftshift_gather(const grid_base_type *in, grid_base_type *out
 }
 
 // Scatter back with fftshift (out[i] = in[(i + (N+1)/2) % N]) and the optional taper division.
+// reals: the float32 real parts go where the in-place layout of fft_and_repacking_routines.cpp:
+// 106-116 wants them, image (f, k) from float index (f*fstride + k) * npix of the buffer on, and
+// a word of the complex image is written unless a real part takes its place.  Every word of
+// the buffer so has one writer, and one pass does what a scatter, an extraction and a copy of
+// the real parts did in three.
 __global__ void k_fftshift_scatter(const grid_base_type *in, grid_base_type *out, uint32_t F,
                                    uint32_t n, uint32_t fstride, uint32_t nx, uint32_t ny,
-                                   const double *tx, const double *ty) {
+                                   const double *tx, const double *ty, int reals) {
     const uint64_t npix = (uint64_t)nx * ny;
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (uint64_t)F * n * npix) return;
@@ -112,45 +118,44 @@ __global__ void k_fftshift_scatter(const grid_base_type *in, grid_base_type *out
     const uint32_t y = (uint32_t)(pix / nx), x = (uint32_t)(pix - (uint64_t)y * nx);
     const uint32_t sy = (y + (ny + 1) / 2) % ny, sx = (x + (nx + 1) / 2) % nx;
     const grid_base_type *src = in + (s * npix + (uint64_t)sy * nx + sx) * 2;
-    grid_base_type re = src[0], im = src[1];
+    grid_base_type v[2] = {src[0], src[1]};
     if (tx) {
         const double t = 1.0 / (tx[x] * ty[y]);
-        re = (grid_base_type)(re * t);
-        im = (grid_base_type)(im * t);
+        v[0] = (grid_base_type)(v[0] * t);
+        v[1] = (grid_base_type)(v[1] * t);
     }
-    grid_base_type *dst = out + (((uint64_t)f * fstride + k) * npix + pix) * 2;
-    dst[0] = re;
-    dst[1] = im;
-}
-
-// Real parts of the first n slices of each facet block -> float32 [F][n][npix]
-__global__ void k_extract_real(const grid_base_type *in, float *tmp, uint32_t F, uint32_t n,
-                               uint32_t fstride, uint64_t npix) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)F * n * npix) return;
-    const uint64_t fn = (uint64_t)n * npix;
-    const uint64_t f = i / fn, j = i - f * fn;
-    tmp[i] = (float)in[(f * fstride * npix + j) * 2];
-}
-
-// float32 images written from float index f*fstride*npix (the in-place layout of
-// fft_and_repacking_routines.cpp:106-116)
-__global__ void k_place_real(const float *tmp, float *out, uint32_t F, uint32_t n,
-                             uint32_t fstride, uint64_t npix) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)F * n * npix) return;
-    const uint64_t fn = (uint64_t)n * npix;
-    const uint64_t f = i / fn, j = i - f * fn;
-    out[f * fstride * npix + j] = tmp[i];
+    const uint64_t block = (uint64_t)fstride * npix;   // floats from one facet's reals to the next's
+    const uint64_t at = (uint64_t)k * npix + pix;
+    if (!reals) {
+        grid_base_type *dst = out + ((uint64_t)f * block + at) * 2;
+        dst[0] = v[0];
+        dst[1] = v[1];
+        return;
+    }
+    constexpr int WORDS = 2 * sizeof(grid_base_type) / 4;   // of a complex value
+    uint32_t w[WORDS];
+    __builtin_memcpy(w, v, sizeof w);
+    uint32_t *words = reinterpret_cast<uint32_t *>(out);
+    words[(uint64_t)f * block + at] = __float_as_uint((float)v[0]);
+#pragma unroll
+    for (int j = 0; j < WORDS; ++j) {
+        // word f * WORDS * block + o: o < WORDS * block lies in the reals' block f * WORDS + q
+        const uint64_t o = at * WORDS + j;
+        uint64_t q = 0;
+#pragma unroll
+        for (int b = 1; b < WORDS; ++b) q += o >= b * block ? 1 : 0;
+        const bool taken = (uint64_t)f * WORDS + q < F && o - q * block < (uint64_t)n * npix;
+        if (!taken) words[(uint64_t)f * WORDS * block + o] = w[j];
+    }
 }
 
 static inline unsigned nblk(uint64_t n) { return (unsigned)((n + 255) / 256); }
 
 hipError_t grid_to_abi(const double *g, void *out, uint64_t slices_fc, uint32_t P,
-                       uint32_t pstride, uint64_t npix, hipStream_t st) {
+                       uint32_t pstride, uint64_t npix, hipStream_t st, const int *err) {
     if (!slices_fc || !npix) return hipSuccess;
     k_grid_to_abi<<<nblk(slices_fc * npix), 256, 0, st>>>(g, (grid_base_type *)out, slices_fc, P,
-                                                         pstride, npix);
+                                                         pstride, npix, err);
     return hipGetLastError();
 }
 
@@ -162,21 +167,58 @@ hipError_t abi_to_grid(const void *in, double *g, uint64_t slices_fc, uint32_t P
     return hipGetLastError();
 }
 
-// Sums the slot copies of an array into slot 0 and clears the others.
-__global__ void k_fold_slots(double *p, uint64_t stride, uint32_t nslots) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= stride) return;
-    double s = p[i];
-    for (uint32_t j = 1; j < nslots; ++j) {
+// Sums the slot copies of an array into slot 0 and clears the others: a wavefront an element, a
+// lane a slot (one thread an element took 16 us for its chain of 64 loads and stores).
+// host: mapped host memory that receives the sums too, unless err is set (nothing is folded
+// then).
+__global__ void k_fold_slots(double *p, uint64_t stride, uint32_t nslots, double *host,
+                             const int *err) {
+    const uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64;
+    if (i >= stride || (err && *err)) return;
+    const uint32_t lane = threadIdx.x & 63;
+    double s = 0.0;
+    for (uint32_t j = lane; j < nslots; j += 64) {
         s += p[(uint64_t)j * stride + i];
-        p[(uint64_t)j * stride + i] = 0.0;
+        if (j) p[(uint64_t)j * stride + i] = 0.0;
     }
-    p[i] = s;
+    s = wave_sum(s);
+    if (lane == 0) {
+        p[i] = s;
+        if (host) host[i] = s;
+    }
 }
 
-hipError_t fold_slots(double *p, uint64_t stride, uint32_t nslots, hipStream_t st) {
-    if (!stride || nslots < 2) return hipSuccess;
-    k_fold_slots<<<nblk(stride), 256, 0, st>>>(p, stride, nslots);
+hipError_t fold_slots(double *p, uint64_t stride, uint32_t nslots, hipStream_t st, double *host,
+                      const int *err) {
+    if (!stride || (nslots < 2 && !host)) return hipSuccess;
+    k_fold_slots<<<nblk(stride * 64), 256, 0, st>>>(p, stride, nslots, host, err);
+    return hipGetLastError();
+}
+
+// What the host reads after a synchronisation, written to mapped host memory by the stream
+// itself (three blocking copies of a few bytes took 30 us each): the error flag, which is
+// cleared, the walk order and the sums of the counter slots.
+__global__ void k_report(int *err, const int *walk, const unsigned long long *counters,
+                         uint32_t nslots, HostReport *out) {
+    const uint32_t lane = threadIdx.x;
+    unsigned long long s = 0, t = 0;
+    for (uint32_t j = lane; j < nslots; j += 64) {
+        s += counters[2 * j];
+        t += counters[2 * j + 1];
+    }
+    s = wave_sum(s);
+    t = wave_sum(t);
+    if (lane) return;
+    out->samples = s;
+    out->taps = t;
+    out->walk = walk ? *walk : 0;
+    out->error = *err;
+    *err = 0;
+}
+
+hipError_t launch_report(int *err, const int *walk, const unsigned long long *counters,
+                         uint32_t nslots, HostReport *out, hipStream_t st) {
+    k_report<<<1, 64, 0, st>>>(err, walk, counters, nslots, out);
     return hipGetLastError();
 }
 
@@ -274,31 +316,74 @@ hipError_t weight_uniformly_device(void *out, const void *sf, const uint64_t *cg
     return hipGetLastError();
 }
 
-// In place on the device buffer `buf` (complex<grid_base_type>, facet blocks of fstride
-// slices): shifts + unnormalised backward FFT + optional taper, then (if place_real) the
-// float32 real parts at the reference's positions.  scratch: F*n*npix complex;
-// rtmp: F*n*npix float.
-hipError_t finalize_device(void *buf, uint32_t F, uint32_t n, uint32_t fstride, uint32_t nx,
-                           uint32_t ny, const double *tx, const double *ty, void *scratch,
-                           float *rtmp, bool place_real, hipStream_t st) {
-    const uint64_t npix = (uint64_t)nx * ny;
-    const uint64_t total = (uint64_t)F * n * npix;
-    if (!total) return hipSuccess;
-    grid_base_type *b = (grid_base_type *)buf;
-    grid_base_type *s = (grid_base_type *)scratch;
-    k_ifftshift_gather<<<nblk(total), 256, 0, st>>>(b, s, F, n, fstride, nx, ny);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipfftHandle plan;
+// FFT plans of the shapes last transformed.  Making one takes 10 to 20 ms (the library builds
+// its kernels for the shape), the transform of a 1024^2 image 40 us.  A context's images and
+// point spread functions need two; the oldest of KEPT leaves for a new shape, and
+// finalize_release_plans gives all back with the context.
+struct FftPlan {
+    hipfftHandle h;
+    uint32_t nx, ny, batch;
+};
+constexpr int KEPT = 4;
+static FftPlan fft_plans[KEPT];
+static int fft_count = 0;
+
+void finalize_release_plans() {
+    for (int i = 0; i < fft_count; ++i) (void)hipfftDestroy(fft_plans[i].h);
+    fft_count = 0;
+}
+
+static hipError_t fft_plan(uint32_t nx, uint32_t ny, uint32_t batch, hipfftHandle *h) {
+    for (int i = 0; i < fft_count; ++i) {
+        const FftPlan &p = fft_plans[i];
+        if (p.nx == nx && p.ny == ny && p.batch == batch) {
+            *h = p.h;
+            return hipSuccess;
+        }
+    }
     int dims[2] = {(int)ny, (int)nx};
+    const int npix = (int)((uint64_t)nx * ny);
 #if defined(BULLSEYE_DOUBLE)
     const hipfftType type = HIPFFT_Z2Z;
 #else
     const hipfftType type = HIPFFT_C2C;
 #endif
-    if (hipfftPlanMany(&plan, 2, dims, nullptr, 1, (int)npix, nullptr, 1, (int)npix, type,
-                       (int)(F * n)) != HIPFFT_SUCCESS)
-        return hipErrorUnknown;
+    FftPlan p = {nullptr, nx, ny, batch};
+    if (hipfftPlanMany(&p.h, 2, dims, nullptr, 1, npix, nullptr, 1, npix, type, (int)batch) !=
+        HIPFFT_SUCCESS) {
+        // the kept plans' work areas may be what is missing
+        finalize_release_plans();
+        if (hipfftPlanMany(&p.h, 2, dims, nullptr, 1, npix, nullptr, 1, npix, type, (int)batch) !=
+            HIPFFT_SUCCESS)
+            return hipErrorUnknown;
+    }
+    if (fft_count == KEPT) {
+        (void)hipfftDestroy(fft_plans[0].h);
+        for (int i = 1; i < KEPT; ++i) fft_plans[i - 1] = fft_plans[i];
+        --fft_count;
+    }
+    fft_plans[fft_count++] = p;
+    *h = p.h;
+    return hipSuccess;
+}
+
+// In place on the device buffer `buf` (complex<grid_base_type>, facet blocks of fstride
+// slices): shifts + unnormalised backward FFT + optional taper, and (if place_real) the float32
+// real parts at the reference's positions.  scratch: F*n*npix complex.  Queued on the stream.
+hipError_t finalize_device(void *buf, uint32_t F, uint32_t n, uint32_t fstride, uint32_t nx,
+                           uint32_t ny, const double *tx, const double *ty, void *scratch,
+                           bool place_real, hipStream_t st) {
+    const uint64_t npix = (uint64_t)nx * ny;
+    const uint64_t total = (uint64_t)F * n * npix;
+    if (!total) return hipSuccess;
+    grid_base_type *b = (grid_base_type *)buf;
+    grid_base_type *s = (grid_base_type *)scratch;
+    hipfftHandle plan;
+    hipError_t e = fft_plan(nx, ny, F * n, &plan);
+    if (e != hipSuccess) return e;
+    k_ifftshift_gather<<<nblk(total), 256, 0, st>>>(b, s, F, n, fstride, nx, ny);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
     hipfftSetStream(plan, st);
 #if defined(BULLSEYE_DOUBLE)
     hipfftResult r = hipfftExecZ2Z(plan, (hipfftDoubleComplex *)s, (hipfftDoubleComplex *)s,
@@ -306,20 +391,10 @@ hipError_t finalize_device(void *buf, uint32_t F, uint32_t n, uint32_t fstride, 
 #else
     hipfftResult r = hipfftExecC2C(plan, (hipfftComplex *)s, (hipfftComplex *)s, HIPFFT_BACKWARD);
 #endif
-    if (r != HIPFFT_SUCCESS) {
-        hipfftDestroy(plan);
-        return hipErrorUnknown;
-    }
-    k_fftshift_scatter<<<nblk(total), 256, 0, st>>>(s, b, F, n, fstride, nx, ny, tx, ty);
-    e = hipGetLastError();
-    if (e == hipSuccess && place_real) {
-        k_extract_real<<<nblk(total), 256, 0, st>>>(b, rtmp, F, n, fstride, npix);
-        k_place_real<<<nblk(total), 256, 0, st>>>(rtmp, (float *)buf, F, n, fstride, npix);
-        e = hipGetLastError();
-    }
-    hipError_t es = hipStreamSynchronize(st);
-    hipfftDestroy(plan);
-    return e != hipSuccess ? e : es;
+    if (r != HIPFFT_SUCCESS) return hipErrorUnknown;
+    k_fftshift_scatter<<<nblk(total), 256, 0, st>>>(s, b, F, n, fstride, nx, ny, tx, ty,
+                                                   place_real ? 1 : 0);
+    return hipGetLastError();
 }
 
 }  // namespace bam

@@ -32,11 +32,20 @@ hipError_t ingest_sort(const uint32_t *a1, const uint32_t *a2, uint32_t rows, ui
                        uint32_t *counts, uint32_t *perm, uint32_t *bl_start, void *ws,
                        size_t ws_bytes, int *err, hipStream_t st);
 hipError_t grid_to_abi(const double *g, void *out, uint64_t slices_fc, uint32_t P,
-                       uint32_t pstride, uint64_t npix, hipStream_t st);
+                       uint32_t pstride, uint64_t npix, hipStream_t st, const int *err = nullptr);
 hipError_t abi_to_grid(const void *in, double *g, uint64_t slices_fc, uint32_t P,
                        uint32_t pstride, uint64_t npix, hipStream_t st);
 hipError_t fill_f64(double *p, uint64_t n, double v, hipStream_t st);
-hipError_t fold_slots(double *p, uint64_t stride, uint32_t nslots, hipStream_t st);
+hipError_t fold_slots(double *p, uint64_t stride, uint32_t nslots, hipStream_t st,
+                      double *host = nullptr, const int *err = nullptr);
+// Mapped host memory a stream reports to before the host waits for it.
+struct HostReport {
+    unsigned long long samples, taps;
+    int walk, error;
+};
+hipError_t launch_report(int *err, const int *walk, const unsigned long long *counters,
+                         uint32_t nslots, HostReport *out, hipStream_t st);
+void finalize_release_plans();
 size_t dft_sample_bytes(uint64_t rows, uint32_t chan);
 hipError_t launch_dft_image(const GridArgs &a, uint64_t rows, void *samples, uint32_t nx,
                             uint32_t ny, double cell_x, double cell_y, double *image,
@@ -53,7 +62,7 @@ hipError_t weight_uniformly_device(void *out, const void *sf, const uint64_t *cg
                                    hipStream_t st);
 hipError_t finalize_device(void *buf, uint32_t F, uint32_t n, uint32_t fstride, uint32_t nx,
                            uint32_t ny, const double *tx, const double *ty, void *scratch,
-                           float *rtmp, bool place_real, hipStream_t st);
+                           bool place_real, hipStream_t st);
 hipError_t fill_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t st);
 hipError_t build_row_tables(const GridArgs &a, uint32_t rows, bool jones, RowRec *rowrec,
                             ChanRec *chanrec, hipStream_t st);

@@ -21,16 +21,17 @@ namespace bam {
 
 
 
-// Two timing events released on every return path.
+// Two timing events, created once and released with the context.
 struct EventPair {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t create() {
-        hipError_t e = hipEventCreate(&e0);
-        return e != hipSuccess ? e : hipEventCreate(&e1);
+        hipError_t e = e0 ? hipSuccess : hipEventCreate(&e0);
+        return e != hipSuccess || e1 ? e : hipEventCreate(&e1);
     }
-    ~EventPair() {
+    void release() {
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
+        e0 = e1 = nullptr;
     }
 };
 
@@ -75,7 +76,7 @@ struct State {
     InputSet ins[2];
     int ins_cur = 0;
     hipStream_t cstream = nullptr;
-    DevBuf out_tmp, fft_scratch, fft_real, jinv, walk, dg_model, dg_out, stokes_tmp, dft_smp,
+    DevBuf out_tmp, fft_scratch, jinv, walk, dg_model, dg_out, stokes_tmp, dft_smp,
         dft_comp;
     // w-projection: taps re-laid per (plane, frac_v, frac_u), per-plane supports and sums
     DevBuf wtaps_f, wtaps_d, wplane_off, wplane_half, wplane_norm, wcls, wlist, wtile;
@@ -86,7 +87,13 @@ struct State {
     std::vector<normalization_base_type> host_norm;
     std::vector<double> taper_x, taper_y;
     // timing
-    std::vector<TimedCall> pending;
+    std::vector<TimedCall> pending, spare;   // spare: events of finished calls, kept for new ones
+    EventPair fin;                           // finalize and degrid timing
+    HostReport *report = nullptr;            // mapped host memory, one
+    double *norm_pin = nullptr;              // mapped host memory, norm_stride
+    bool queued = false;   // work on the stream since the last barrier
+    bool sticky = false;   // bullseye_grid_noalloc was called: its calls may be replayed by a
+                           // graph, so every barrier reads the error flag
     double grid_seconds = 0, inv_seconds = 0;
     bullseye_stats stats{};
     unsigned long long last_counters[2] = {0, 0};
@@ -183,16 +190,8 @@ static size_t psf_elems() { return g.F * g.sfC * g.ny * g.nx * 2; }
 static size_t abi_grid_bytes() { return g.F * g.cube * g.P * g.ny * g.nx * 2 * sizeof(grid_base_type); }
 static size_t abi_psf_bytes() { return g.F * g.sfC * g.ny * g.nx * 2 * sizeof(grid_base_type); }
 
-int check_device_errors() {
-    int flag = 0;
-    if (g.errflag.p) {
-        hipError_t e = hipMemcpy(&flag, g.errflag.p, sizeof(int), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) return fail("reading the device error flag: %s", hipGetErrorString(e));
-        if (flag) {
-            int zero = 0;
-            (void)hipMemcpy(g.errflag.p, &zero, sizeof(int), hipMemcpyHostToDevice);
-        }
-    }
+// The error of a device error flag, as a message.
+static int flag_error(int flag) {
     if (flag & 1) return fail("JONES MATRIX SET CONTAINS SINGULAR MATRICIES");
     if (flag & 2) return fail("antenna id out of range (antenna_count or baseline_count too small)");
     if (flag & 4) return fail("channel grid index, spw id or timestamp id out of range");
@@ -202,15 +201,40 @@ int check_device_errors() {
     return 0;
 }
 
-static int barrier_impl() {
-    if (!g.stream) return 0;
+// Queue the stream's report, wait for the stream, and return the error it reports.
+static int report_and_wait() {
+    HIP_TRY(launch_report(g.errflag.as<int>(), g.walk.as<int>(),
+                          g.counters.as<unsigned long long>(), g.nslots, g.report, g.stream));
     hipError_t e = hipStreamSynchronize(g.stream);
     if (e != hipSuccess) return fail("gridding stream failed: %s", hipGetErrorString(e));
+    g.queued = false;
+    return 0;
+}
+
+int check_device_errors() {
+    if (!g.report) return 0;
+    if (report_and_wait()) return 1;
+    return flag_error(g.report->error);
+}
+
+constexpr size_t SPARE_CALLS = 16;
+
+static void destroy_call(const TimedCall &c) {
+    for (hipEvent_t ev : {c.start, c.cstart, c.copied, c.k0, c.k1, c.stop})
+        if (ev) (void)hipEventDestroy(ev);
+}
+
+// Waits for queued work, takes the timings and counters of the calls since the last barrier, and
+// returns their errors.  Nothing queued: nothing to wait for.
+static int barrier_impl() {
+    if (!g.stream || !g.report) return 0;
+    if (!g.queued && !g.sticky && g.pending.empty()) return 0;
+    if (report_and_wait()) return 1;
+    const HostReport rep = *g.report;
     for (auto &c : g.pending) {
         float ms = 0, kms = 0;
         if (!c.recorded) {
-            for (hipEvent_t ev : {c.start, c.cstart, c.copied, c.k0, c.k1, c.stop})
-                if (ev) (void)hipEventDestroy(ev);
+            destroy_call(c);
             continue;
         }
         (void)hipEventElapsedTime(&ms, c.start, c.stop);
@@ -225,72 +249,49 @@ static int barrier_impl() {
             (void)hipEventElapsedTime(&pms, c.start, c.k0);
             g.stats.prep_ms = pms;
         }
-        (void)hipEventDestroy(c.start);
-        (void)hipEventDestroy(c.cstart);
-        (void)hipEventDestroy(c.copied);
-        (void)hipEventDestroy(c.k0);
-        (void)hipEventDestroy(c.k1);
-        (void)hipEventDestroy(c.stop);
+        c.recorded = c.has_kernel = false;
+        if (g.spare.size() < SPARE_CALLS)
+            g.spare.push_back(c);
+        else
+            destroy_call(c);
     }
     const bool had_pending = !g.pending.empty();
     g.pending.clear();
-    if (had_pending && g.counters.p) {
-        std::vector<unsigned long long> cs(2 * (size_t)g.nslots);
-        e = hipMemcpy(cs.data(), g.counters.p, cs.size() * sizeof(unsigned long long),
-                      hipMemcpyDeviceToHost);
-        if (e != hipSuccess) return fail("reading counters: %s", hipGetErrorString(e));
-        unsigned long long c[2] = {0, 0};
-        for (size_t i = 0; i < g.nslots; ++i) {
-            c[0] += cs[2 * i];
-            c[1] += cs[2 * i + 1];
-        }
-        g.stats.samples_gridded = c[0] - g.last_counters[0];
-        g.stats.taps = c[1] - g.last_counters[1];
-        g.last_counters[0] = c[0];
-        g.last_counters[1] = c[1];
-        if (g.walk.p) {
-            int ti = 0;
-            e = hipMemcpy(&ti, g.walk.p, sizeof ti, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) return fail("reading the walk order: %s", hipGetErrorString(e));
-            g.stats.time_inner = (uint32_t)ti;
-        }
+    if (had_pending) {
+        g.stats.samples_gridded = rep.samples - g.last_counters[0];
+        g.stats.taps = rep.taps - g.last_counters[1];
+        g.last_counters[0] = rep.samples;
+        g.last_counters[1] = rep.taps;
+        if (g.walk.p) g.stats.time_inner = (uint32_t)rep.walk;
     }
-    return check_device_errors();
+    return flag_error(rep.error);
 }
 
-// The device results of all chunks so far, copied into the caller's buffers (final chunk).
-static int publish_results(gridding_parameters *p, bool psf) {
-    if (!psf) {
-        void *dst = dev_mode() ? p->output_buffer : nullptr;
-        if (!dev_mode()) {
-            HIP_TRY(g.out_tmp.ensure(abi_grid_bytes()));
-            dst = g.out_tmp.p;
-        }
-        if (dst)
-            HIP_TRY(grid_to_abi(g.grid.as<double>(), dst, g.F * g.cube, (uint32_t)g.P,
-                                (uint32_t)g.pstride, g.nx * g.ny, g.stream));
-        HIP_TRY(fold_slots(g.norm.as<double>(), g.norm_stride, g.nslots, g.stream));
-        HIP_TRY(hipMemcpyAsync(g.host_norm.data(), g.norm.p,
-                               g.host_norm.size() * sizeof(normalization_base_type),
-                               hipMemcpyDeviceToHost, g.stream));
-        HIP_TRY(hipStreamSynchronize(g.stream));
-        if (!dev_mode() && p->output_buffer)
-            HIP_TRY(hipMemcpy(p->output_buffer, g.out_tmp.p, abi_grid_bytes(),
-                              hipMemcpyDeviceToHost));
-    } else {
-        void *dst = dev_mode() ? p->sampling_function_buffer : nullptr;
-        if (!dev_mode()) {
-            HIP_TRY(g.out_tmp.ensure(std::max(abi_psf_bytes(), g.out_tmp.bytes)));
-            dst = g.out_tmp.p;
-        }
-        if (dst)
-            HIP_TRY(grid_to_abi(g.psfgrid.as<double>(), dst, g.F * g.sfC, 1, 1, g.nx * g.ny,
-                                g.stream));
-        HIP_TRY(hipStreamSynchronize(g.stream));
-        if (!dev_mode() && p->sampling_function_buffer)
-            HIP_TRY(hipMemcpy(p->sampling_function_buffer, g.out_tmp.p, abi_psf_bytes(),
-                              hipMemcpyDeviceToHost));
+// The device results of all chunks so far into the caller's buffers (final chunk): queued behind
+// the gridding, skipped on the device when a call raised an error, with one wait for all of it.
+static int finish_chunks(gridding_parameters *p, bool psf) {
+    void *const caller = psf ? p->sampling_function_buffer : p->output_buffer;
+    const size_t bytes = psf ? abi_psf_bytes() : abi_grid_bytes();
+    void *dst = caller;
+    const int *err = g.errflag.as<int>();
+    if (!dev_mode()) {
+        HIP_TRY(g.out_tmp.ensure(std::max(bytes, g.out_tmp.bytes)));
+        dst = g.out_tmp.p;
     }
+    g.queued = true;
+    if (dst) {
+        if (psf)
+            HIP_TRY(grid_to_abi(g.psfgrid.as<double>(), dst, g.F * g.sfC, 1, 1, g.nx * g.ny,
+                                g.stream, err));
+        else
+            HIP_TRY(grid_to_abi(g.grid.as<double>(), dst, g.F * g.cube, (uint32_t)g.P,
+                                (uint32_t)g.pstride, g.nx * g.ny, g.stream, err));
+    }
+    if (!psf)
+        HIP_TRY(fold_slots(g.norm.as<double>(), g.norm_stride, g.nslots, g.stream, g.norm_pin, err));
+    if (barrier_impl()) return 1;
+    if (!psf) std::copy(g.norm_pin, g.norm_pin + g.norm_stride, g.host_norm.begin());
+    if (!dev_mode() && caller) HIP_TRY(hipMemcpy(caller, dst, bytes, hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -635,17 +636,22 @@ static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
     TimedCall none{};
     TimedCall *tcp = &none;
     if (!noalloc) {
-        g.pending.push_back(TimedCall{});
-        tcp = &g.pending.back();
-        HIP_TRY(hipEventCreate(&tcp->start));
-        HIP_TRY(hipEventCreate(&tcp->cstart));
-        HIP_TRY(hipEventCreate(&tcp->copied));
-        HIP_TRY(hipEventCreate(&tcp->k0));
-        HIP_TRY(hipEventCreate(&tcp->k1));
-        HIP_TRY(hipEventCreate(&tcp->stop));
+        if (g.spare.empty()) {
+            g.pending.push_back(TimedCall{});
+            tcp = &g.pending.back();
+            for (hipEvent_t *ev : {&tcp->start, &tcp->cstart, &tcp->copied, &tcp->k0, &tcp->k1,
+                                   &tcp->stop})
+                HIP_TRY(hipEventCreate(ev));
+        } else {
+            g.pending.push_back(g.spare.back());
+            g.spare.pop_back();
+            tcp = &g.pending.back();
+        }
         HIP_TRY(hipEventRecord(tcp->start, g.stream));
     }
     TimedCall &tc = *tcp;
+    g.queued = true;
+    g.sticky |= noalloc;
 
     GridArgs a{};
     if (setup_inputs(p, mode, facet, phase, psf, true, a, tc.cstart, tc.copied)) return 1;
@@ -744,11 +750,7 @@ static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
         HIP_TRY(hipEventRecord(tc.stop, g.stream));
         tc.recorded = true;
     }
-    if (p->is_final_data_chunk) {
-        if (barrier_impl()) return 1;
-        if (publish_results(p, psf)) return 1;
-    }
-    return 0;
+    return p->is_final_data_chunk ? finish_chunks(p, psf) : 0;
 }
 
 // W-projection taps: conv[plane][csz][csz] complex -> contiguous W_p x W_p blocks per
@@ -935,7 +937,7 @@ int bullseye_reset_grids(void) {
     HIP_TRY(fill_f64(g.grid.as<double>(), grid_elems(), 0.0, g.stream));
     if (g.psf) HIP_TRY(fill_f64(g.psfgrid.as<double>(), psf_elems(), 0.0, g.stream));
     HIP_TRY(fill_f64(g.norm.as<double>(), g.norm_stride * g.nslots, 0.0, g.stream));
-    HIP_TRY(hipStreamSynchronize(g.stream));
+    g.queued = true;   // what follows on the stream is ordered behind it
     std::fill(g.host_norm.begin(), g.host_norm.end(), 0.0);
     return 0;
 }
@@ -952,7 +954,7 @@ static void release_resources() {
                       &g.geom, &g.taper, &g.perm, &g.blstart, &g.keys, &g.vals, &g.keys_out,
                       &g.rowrec, &g.chanrec,
                       &g.counts, &g.ws, &g.out_tmp,
-                      &g.fft_scratch, &g.fft_real, &g.jinv, &g.wtaps_f, &g.wtaps_d,
+                      &g.fft_scratch, &g.jinv, &g.wtaps_f, &g.wtaps_d,
                       &g.wplane_off, &g.wplane_half, &g.wplane_norm, &g.wcls, &g.wlist, &g.wtile, &g.walk,
                       &g.wctaps_f, &g.wctaps_d, &g.wcplane_off,
                       &g.dg_model, &g.dg_out, &g.stokes_tmp, &g.dft_smp, &g.dft_comp};
@@ -969,6 +971,17 @@ static void release_resources() {
     if (g.cstream) (void)hipStreamDestroy(g.cstream);
     g.cstream = nullptr;
     batch_release_all();
+    finalize_release_plans();
+    for (const TimedCall &c : g.pending) destroy_call(c);
+    for (const TimedCall &c : g.spare) destroy_call(c);
+    g.pending.clear();
+    g.spare.clear();
+    g.fin.release();
+    if (g.report) (void)hipHostFree(g.report);
+    if (g.norm_pin) (void)hipHostFree(g.norm_pin);
+    g.report = nullptr;
+    g.norm_pin = nullptr;
+    g.queued = g.sticky = false;
     for (int i = 0; i < State::WSIDE; ++i) {
         if (g.wside[i]) (void)hipStreamDestroy(g.wside[i]);
         if (g.wjoin[i]) (void)hipEventDestroy(g.wjoin[i]);
@@ -1041,6 +1054,9 @@ static int init_impl(gridding_parameters *p) {
     HIP_TRY(g.norm.ensure(g.norm_stride * g.nslots * sizeof(double)));
     HIP_TRY(g.counters.ensure(2 * (size_t)g.nslots * sizeof(unsigned long long)));
     HIP_TRY(g.errflag.ensure(sizeof(int)));
+    HIP_TRY(hipHostMalloc((void **)&g.report, sizeof(HostReport), hipHostMallocMapped));
+    HIP_TRY(hipHostMalloc((void **)&g.norm_pin, g.norm_stride * sizeof(double),
+                          hipHostMallocMapped));
     HIP_TRY(hipMemset(g.counters.p, 0, 2 * (size_t)g.nslots * sizeof(unsigned long long)));
     HIP_TRY(hipMemset(g.errflag.p, 0, sizeof(int)));
     g.last_counters[0] = g.last_counters[1] = 0;
@@ -1222,7 +1238,7 @@ static int finalize_impl(gridding_parameters *p, bool psf) {
                                             : p->cube_channel_dim_size * g.P);
     const size_t npix = p->nx * p->ny;
     const size_t total_bytes = (size_t)F * fstride * npix * 2 * sizeof(grid_base_type);
-    EventPair ev;
+    EventPair &ev = g.fin;
     HIP_TRY(ev.create());
     HIP_TRY(hipEventRecord(ev.e0, g.stream));
     void *dbuf = buf;
@@ -1232,12 +1248,11 @@ static int finalize_impl(gridding_parameters *p, bool psf) {
         dbuf = g.out_tmp.p;
     }
     HIP_TRY(g.fft_scratch.ensure((size_t)F * n * npix * 2 * sizeof(grid_base_type)));
-    HIP_TRY(g.fft_real.ensure((size_t)F * n * npix * sizeof(float)));
     const bool taper = g.opts.apply_taper_correction && !psf && g.taper.p;
     const double *tx = taper ? g.taper.as<double>() : nullptr;
     const double *ty = taper ? g.taper.as<double>() + g.nx : nullptr;
     HIP_TRY(finalize_device(dbuf, F, n, fstride, (uint32_t)p->nx, (uint32_t)p->ny, tx, ty,
-                            g.fft_scratch.p, g.fft_real.as<float>(), dev_mode(), g.stream));
+                            g.fft_scratch.p, dev_mode(), g.stream));
     HIP_TRY(hipEventRecord(ev.e1, g.stream));
     HIP_TRY(hipEventSynchronize(ev.e1));
     float ms = 0;
@@ -1389,6 +1404,7 @@ int bullseye_dft_image(gridding_parameters *p, double *image) {
     if (!p || !image) return fail("bullseye_dft_image: NULL argument");
     if (validate_call(p, MODE_1)) return 1;
     if (barrier_impl()) return 1;
+    g.queued = true;
     GridArgs a{};
     if (setup_inputs(p, MODE_1, false, false, false, true, a)) return 1;
     const uint64_t rows = p->row_count, npix = (uint64_t)p->nx * p->ny;
@@ -1404,7 +1420,6 @@ int bullseye_dft_image(gridding_parameters *p, double *image) {
                              g.stream));
     if (!dev_mode())
         HIP_TRY(hipMemcpyAsync(image, dimg, npix * sizeof(double), hipMemcpyDeviceToHost, g.stream));
-    HIP_TRY(hipStreamSynchronize(g.stream));
     return check_device_errors();
 }
 
@@ -1415,6 +1430,7 @@ int bullseye_dft_predict(gridding_parameters *p, const double *components, uint3
     if (!p || !vis_out || (n && !components)) return fail("bullseye_dft_predict: NULL argument");
     if (validate_call(p, MODE_1)) return 1;
     if (barrier_impl()) return 1;
+    g.queued = true;
     GridArgs a{};
     if (setup_inputs(p, MODE_1, false, false, false, false, a)) return 1;
     const uint64_t rows = p->row_count;
@@ -1435,7 +1451,6 @@ int bullseye_dft_predict(gridding_parameters *p, const double *components, uint3
     HIP_TRY(launch_dft_predict(a, rows, dcomp, n, dvis, g.stream));
     if (!dev_mode())
         HIP_TRY(hipMemcpyAsync(vis_out, dvis, vbytes, hipMemcpyDeviceToHost, g.stream));
-    HIP_TRY(hipStreamSynchronize(g.stream));
     return check_device_errors();
 }
 
@@ -1454,8 +1469,9 @@ int bullseye_degrid(gridding_parameters *p, int mode, const void *model, void *v
     const size_t rows = p->row_count, C = p->channel_count, npol = p->number_of_polarization_terms;
     const size_t model_bytes = g.F * g.cube * g.P * g.ny * g.nx * 2 * sizeof(grid_base_type);
     const size_t out_bytes = rows * C * npol * 2 * sizeof(visibility_base_type);
-    EventPair ev;
+    EventPair &ev = g.fin;
     HIP_TRY(ev.create());
+    g.queued = true;
     GridArgs a{};
     if (setup_inputs(p, km, modes[mode].facet, modes[mode].phase, false, false, a)) return 1;
     const void *dm = model;
@@ -1477,11 +1493,11 @@ int bullseye_degrid(gridding_parameters *p, int mode, const void *model, void *v
     HIP_TRY(hipEventRecord(ev.e1, g.stream));
     if (!dev_mode())
         HIP_TRY(hipMemcpyAsync(vis_out, dout, out_bytes, hipMemcpyDeviceToHost, g.stream));
-    HIP_TRY(hipStreamSynchronize(g.stream));
+    const int rc = check_device_errors();
     float ms = 0;
-    (void)hipEventElapsedTime(&ms, ev.e0, ev.e1);
+    if (!rc) (void)hipEventElapsedTime(&ms, ev.e0, ev.e1);
     g.stats.kernel_ms = ms;
-    return check_device_errors();
+    return rc;
 }
 
 }  // extern "C"
