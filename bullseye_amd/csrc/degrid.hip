@@ -11,16 +11,25 @@
 //   S = Pinv^H S Qinv in the Jones mode (the forward applies V -> Pinv V Qinv^H),
 // and out[row][chan][corr_k] = sum over facets of s_k; every other correlation is zero.
 //
-// A gather: no atomics.  A group of GL lanes shares one (row, channel) sample and splits the
-// footprint's taps; a butterfly over the group's lanes combines the partial sums.  Neighbouring
-// samples of a row read overlapping grid rows, which stay in L2.
+// A gather: no atomics.  One lane prepares one (row, channel) sample per facet (the FP64 geometry
+// and rotor, 200 instructions, once: a group of 16 lanes sharing a sample repeated them 16
+// times and was bound by that).  The taps are then summed
+//   AA, W = 3..11   by the sample's own lane: both tap runs in registers, the model read in
+//                   rows of W complex values; neighbouring lanes are neighbouring channels, whose
+//                   footprints share cache lines.  9 instructions a sample's tap row and
+//                   correlation, and no exchange between lanes (6 facets x 4 correlations,
+//                   1.01 M samples: 1.69 -> 0.38 ms a call).
+//   others          by the wavefront, sample after sample: a sample's w-kernel block is W_p x W_p
+//                   consecutive taps, which lanes of their own samples could only read line by
+//                   line.  Eight samples' partial sums are reduced together (each exchange halves
+//                   the samples a lane keeps: 10 exchanges for eight, not 6 for each).
 #include "device_common.h"
 
 namespace bam {
 namespace dg {
 
-constexpr int GL = 16;      // lanes per sample
 constexpr int BLOCK = 256;
+constexpr int PACK = 8;     // samples reduced together
 
 struct DArgs {
     GridArgs g;                      // inputs and geometry (g.grid and g.norm unused)
@@ -35,226 +44,381 @@ struct DArgs {
     uint64_t rows;
 };
 
-template <typename T> __device__ __forceinline__ T group_sum(T v) {
+// One sample: what does not depend on the facet.
+template <int MODE, int PATH> struct Sample {
+    static constexpr int NC = ModeTraits<MODE>::NCORR;
+    typedef typename PathTraits<PATH>::acc_t T;
+    bool in_range, live;
+    uint32_t row, c, s;
+    uint64_t cgi;
+    size_t base;
+    T wt[NC];
+    size_t jb1, jb2;
+    double u, v, w;
+
+    // the checks are the forward's, in its order
+    __device__ __forceinline__ void load(const DArgs &d, uint64_t sample) {
+        const GridArgs &a = d.g;
+        in_range = sample < d.rows * a.chan;
+        row = in_range ? (uint32_t)(sample / a.chan) : 0;
+        c = in_range ? (uint32_t)(sample % a.chan) : 0;
+        base = ((size_t)row * a.chan + c) * a.npol;
+        live = in_range;
+        s = 0;
+        cgi = 0;
+        jb1 = jb2 = 0;
+        u = v = w = 0;
 #pragma unroll
-    for (int o = GL / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, GL);
-    return v;
+        for (int k = 0; k < NC; ++k) wt[k] = T(0);
+        if (live) {
+            s = a.spw[row];
+            if (s >= a.spw_count) {
+                atomicOr(a.error_flag, 4);
+                live = false;
+            }
+        }
+        if (live && !a.enabled[s * a.chan + c]) live = false;
+        if (live) {
+            cgi = a.cgi[s * a.chan + c];
+            if (cgi >= a.cube) {
+                atomicOr(a.error_flag, 4);
+                live = false;
+            }
+        }
+        if (live && (a.row_flags[row] || a.field[row] != a.imaging_field)) live = false;
+        if (live) {
+            bool any = false;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                const size_t idx = base + a.pol_idx[k];
+                wt[k] = a.flags[idx] ? T(0) : (T)a.weights[idx];
+                any |= wt[k] != T(0);
+            }
+            live = any;
+        }
+        if constexpr (MODE == MODE_4J) {
+            if (live) {
+                const size_t t = a.time_ids[row];
+                if (t >= a.ntime || a.ant1[row] >= a.antenna_count ||
+                    a.ant2[row] >= a.antenna_count) {
+                    atomicOr(a.error_flag, 4);
+                    live = false;
+                } else {
+                    jb1 = ((size_t)t * a.antenna_count + a.ant1[row]) * a.facets;
+                    jb2 = ((size_t)t * a.antenna_count + a.ant2[row]) * a.facets;
+                }
+            }
+        }
+        if (live) {
+            const double rw = 1.0 / (double)a.wavelengths[s * a.chan + c];
+            u = (double)a.uvw[3 * (size_t)row] * rw;
+            v = (double)a.uvw[3 * (size_t)row + 1] * rw;
+            w = (double)a.uvw[3 * (size_t)row + 2] * rw;
+        }
+    }
+};
+
+// Place of a sample on a facet's grid.
+template <typename T> struct Place {
+    bool on, conj;
+    T cs, sn;              // the forward's rotor
+    int x0, y0, fu, fv, wp;
+    uint32_t tb;
+};
+
+template <int MODE, int PATH, bool WPROJ>
+__device__ __forceinline__ Place<typename PathTraits<PATH>::acc_t>
+place(const DArgs &d, const Sample<MODE, PATH> &sm, uint32_t f) {
+    typedef typename PathTraits<PATH>::acc_t T;
+    const GridArgs &a = d.g;
+    const FacetGeom *gp = a.geom + f;
+    Place<T> p = {sm.live, false, T(1), T(0), 0, 0, 0, 0, 0, 0};
+    double u = sm.u, v = sm.v, w = sm.w;
+    if (p.on && a.phase) {  // the forward's rotor, in turns, FP64 argument
+        const double turns = u * gp->dl + v * gp->dm + w * gp->dn;
+        const double fr = 2.0 * (turns - rint(turns));
+        if constexpr (PATH == PATH_FP64) {
+            double s_, c_;
+            sincospi(fr, &s_, &c_);
+            p.sn = s_;
+            p.cs = c_;
+        } else {
+            float s_, c_;
+            sincospi_unit((float)fr, &s_, &c_);
+            p.sn = s_;
+            p.cs = c_;
+        }
+    }
+    if (a.transform) {
+        u = u - w * gp->u_term;
+        v = v - w * gp->v_term;
+    }
+    u *= a.u_scale;
+    v *= a.v_scale;
+    if constexpr (!WPROJ) {  // AA tap choice under the forward's floor rounding
+        const double flu = floor(u), flv = floor(v);
+        p.x0 = (int)flu + (int)a.off_x;
+        p.y0 = (int)flv + (int)a.off_y;
+        p.fu = (int)((1.0 - u + flu) * a.OS);
+        p.fv = (int)((1.0 - v + flv) * a.OS);
+        p.wp = (int)a.W;
+        if (p.x0 < 0 || p.y0 < 0 || p.x0 >= (int)a.nx - p.wp - 2 || p.y0 >= (int)a.ny - p.wp - 2)
+            p.on = false;
+    } else {  // w-projection: w < 0 conjugation, nearest rounding, plane choice
+        if (w < 0) {
+            p.conj = true;
+            u = -u;
+            v = -v;
+            w = -w;
+        }
+        const double ru = rint(u), rv = rint(v);
+        const int dx = (int)rint(u + a.off_x), dy = (int)rint(v + a.off_y);
+        const int fu = (int)((1.0 - u + ru) * a.OS) - (int)d.fbase;
+        const int fv = (int)((1.0 - v + rv) * a.OS) - (int)d.fbase;
+        const double pl = rint(w / (double)d.wmax_f * (double)(d.wplanes - 1));
+        const int padded = 2 * (int)a.S + 3;
+        if (dx < 0 || dy < 0 || dx >= (int)a.nx - padded || dy >= (int)a.ny - padded ||
+            pl >= (double)d.wplanes || (uint32_t)fu >= d.nf || (uint32_t)fv >= d.nf)
+            p.on = false;
+        if (p.on) {
+            const int plane = (int)pl;
+            const int sp = (int)d.plane_half[plane];
+            p.wp = 2 * sp + 1;
+            p.x0 = dx + (int)a.S - sp;
+            p.y0 = dy + (int)a.S - sp;
+            p.tb = (uint32_t)(d.plane_off[plane] +
+                              ((uint64_t)fv * d.nf + (uint64_t)fu) * (uint64_t)(p.wp * p.wp));
+        }
+    }
+    return p;
 }
 
+// The sample's footprint sums to its visibilities: conjugation, rotor, weights, Jones terms.
 template <int MODE, int PATH>
-__global__ __launch_bounds__(BLOCK) void degrid_kernel(DArgs d) {
+__device__ __forceinline__ void finish(const DArgs &d, const Sample<MODE, PATH> &sm,
+                                       const Place<typename PathTraits<PATH>::acc_t> &p, uint32_t f,
+                                       cpx<typename PathTraits<PATH>::acc_t> (&sk)[ModeTraits<MODE>::NCORR],
+                                       cpx<typename PathTraits<PATH>::acc_t> (&acc)[ModeTraits<MODE>::NCORR]) {
     constexpr int NC = ModeTraits<MODE>::NCORR;
     typedef typename PathTraits<PATH>::acc_t T;
     const GridArgs &a = d.g;
-    const uint64_t sample = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) / GL;
-    const int gl = (int)(threadIdx.x % GL);
-    const bool in_range = sample < d.rows * a.chan;
-    const uint32_t row = in_range ? (uint32_t)(sample / a.chan) : 0;
-    const uint32_t c = in_range ? (uint32_t)(sample % a.chan) : 0;
-    const size_t base = ((size_t)row * a.chan + c) * a.npol;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        if (p.conj) sk[k] = conjg(sk[k]);
+        sk[k] = cmul(sk[k], cpx<T>{p.cs, -p.sn});
+        sk[k].re *= sm.wt[k];
+        sk[k].im *= sm.wt[k];
+    }
+    if constexpr (MODE == MODE_4J) {  // S = Pinv^H S Qinv
+        const size_t j1 = ((sm.jb1 + f) * a.spw_count + sm.s) * a.chan + sm.c;
+        const size_t j2 = ((sm.jb2 + f) * a.spw_count + sm.s) * a.chan + sm.c;
+        const cpx<T> *A = reinterpret_cast<const cpx<T> *>(a.jones_inv) + 4 * j1;
+        const cpx<T> *B = reinterpret_cast<const cpx<T> *>(a.jones_inv) + 4 * j2;
+        const cpx<T> a0 = conjg(A[0]), a1 = conjg(A[1]), a2 = conjg(A[2]), a3 = conjg(A[3]);
+        const cpx<T> t0 = cadd(cmul(a0, sk[0]), cmul(a2, sk[2]));
+        const cpx<T> t1 = cadd(cmul(a0, sk[1]), cmul(a2, sk[3]));
+        const cpx<T> t2 = cadd(cmul(a1, sk[0]), cmul(a3, sk[2]));
+        const cpx<T> t3 = cadd(cmul(a1, sk[1]), cmul(a3, sk[3]));
+        sk[0] = cadd(cmul(t0, B[0]), cmul(t1, B[2]));
+        sk[1] = cadd(cmul(t0, B[1]), cmul(t1, B[3]));
+        sk[2] = cadd(cmul(t2, B[0]), cmul(t3, B[2]));
+        sk[3] = cadd(cmul(t2, B[1]), cmul(t3, B[3]));
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[k] = cadd(acc[k], sk[k]);
+}
 
-    // per-sample checks, in the forward's order (every lane of the group agrees)
-    bool live = in_range;
-    uint32_t s = 0;
-    uint64_t cgi = 0;
-    if (live) {
-        s = a.spw[row];
-        if (s >= a.spw_count) {
-            if (gl == 0) atomicOr(a.error_flag, 4);
-            live = false;
-        }
-    }
-    if (live && !a.enabled[s * a.chan + c]) live = false;
-    if (live) {
-        cgi = a.cgi[s * a.chan + c];
-        if (cgi >= a.cube) {
-            if (gl == 0) atomicOr(a.error_flag, 4);
-            live = false;
-        }
-    }
-    if (live && (a.row_flags[row] || a.field[row] != a.imaging_field)) live = false;
-    T wt[NC];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) wt[k] = T(0);
-    if (live) {
-        bool any = false;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            const size_t idx = base + a.pol_idx[k];
-            wt[k] = a.flags[idx] ? T(0) : (T)a.weights[idx];
-            any |= wt[k] != T(0);
-        }
-        live = any;
-    }
-    size_t jb1 = 0, jb2 = 0;
-    if constexpr (MODE == MODE_4J) {
-        if (live) {
-            const size_t t = a.time_ids[row];
-            if (t >= a.ntime || a.ant1[row] >= a.antenna_count ||
-                a.ant2[row] >= a.antenna_count) {
-                if (gl == 0) atomicOr(a.error_flag, 4);
-                live = false;
-            } else {
-                jb1 = ((size_t)t * a.antenna_count + a.ant1[row]) * a.facets;
-                jb2 = ((size_t)t * a.antenna_count + a.ant2[row]) * a.facets;
-            }
-        }
-    }
-    double u0 = 0, v0 = 0, w0 = 0;
-    if (live) {
-        const double rw = 1.0 / (double)a.wavelengths[s * a.chan + c];
-        u0 = (double)a.uvw[3 * (size_t)row] * rw;
-        v0 = (double)a.uvw[3 * (size_t)row + 1] * rw;
-        w0 = (double)a.uvw[3 * (size_t)row + 2] * rw;
-    }
-
-    const size_t slice = (size_t)a.nx * a.ny;
-    const T *conv = reinterpret_cast<const T *>(a.conv);
-    const cpx<T> *wtaps = reinterpret_cast<const cpx<T> *>(d.taps);
-    const int padded = 2 * (int)a.S + 3;
-    cpx<T> acc[NC];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) acc[k] = {T(0), T(0)};
-
-    for (uint32_t f = 0; f < a.facets; ++f) {
-        bool on = live;
-        const FacetGeom *gp = a.geom + f;
-        double u = u0, v = v0, w = w0;
-        T cs = T(1), sn = T(0);
-        if (on && a.phase) {  // the forward's rotor, in turns, FP64 argument
-            const double turns = u * gp->dl + v * gp->dm + w * gp->dn;
-            const double fr = 2.0 * (turns - rint(turns));
-            if constexpr (PATH == PATH_FP64) {
-                double s_, c_;
-                sincospi(fr, &s_, &c_);
-                sn = s_;
-                cs = c_;
-            } else {
-                float s_, c_;
-                sincospif((float)fr, &s_, &c_);
-                sn = s_;
-                cs = c_;
-            }
-        }
-        if (a.transform) {
-            u = u - w * gp->u_term;
-            v = v - w * gp->v_term;
-        }
-        u *= a.u_scale;
-        v *= a.v_scale;
-        bool conj_out = false;
-        int x0 = 0, y0 = 0, fu = 0, fv = 0, wp = 0;
-        uint32_t tb = 0;
-        if (!d.wproj) {  // AA tap choice under the forward's floor rounding
-            const double flu = floor(u), flv = floor(v);
-            x0 = (int)flu + (int)a.off_x;
-            y0 = (int)flv + (int)a.off_y;
-            fu = (int)((1.0 - u + flu) * a.OS);
-            fv = (int)((1.0 - v + flv) * a.OS);
-            wp = (int)a.W;
-            if (x0 < 0 || y0 < 0 || x0 + wp + 2 >= (int)a.nx || y0 + wp + 2 >= (int)a.ny)
-                on = false;
-        } else {  // w-projection: w < 0 conjugation, nearest rounding, plane choice
-            if (w < 0) {
-                conj_out = true;
-                u = -u;
-                v = -v;
-                w = -w;
-            }
-            const double ru = rint(u), rv = rint(v);
-            const int dx = (int)rint(u + a.off_x), dy = (int)rint(v + a.off_y);
-            fu = (int)((1.0 - u + ru) * a.OS);
-            fv = (int)((1.0 - v + rv) * a.OS);
-            const double pl = rint(w / (double)d.wmax_f * (double)(d.wplanes - 1));
-            if (dx < 0 || dy < 0 || dx + padded >= (int)a.nx || dy + padded >= (int)a.ny ||
-                pl >= (double)d.wplanes)
-                on = false;
-            if (on) {
-                const int plane = (int)pl;
-                const int sp = (int)d.plane_half[plane];
-                wp = 2 * sp + 1;
-                x0 = dx + (int)a.S - sp;
-                y0 = dy + (int)a.S - sp;
-                tb = (uint32_t)(d.plane_off[plane] +
-                                ((uint64_t)(fv - (int)d.fbase) * d.nf + (uint64_t)(fu - (int)d.fbase)) *
-                                    (uint64_t)(wp * wp));
-            }
-        }
-        cpx<T> sk[NC];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) sk[k] = {T(0), T(0)};
-        if (on) {
-            const grid_base_type *gb = d.model + ((size_t)f * a.cube + cgi) * d.P * slice * 2;
-            const int ntap = wp * wp;
-            for (int t = gl; t < ntap; t += GL) {
-                const int j = t / wp, k = t - j * wp;
-                cpx<T> tap;
-                if (!d.wproj) {
-                    tap = {conv[fu + k * (int)a.OS] * conv[fv + j * (int)a.OS], T(0)};
-                } else {
-                    const cpx<T> tw = wtaps[tb + (uint32_t)t];
-                    tap = {tw.re, -tw.im};
-                }
-                const size_t pos = (size_t)(y0 + j) * a.nx + (size_t)(x0 + k);
-#pragma unroll
-                for (int kk = 0; kk < NC; ++kk) {
-                    const grid_base_type *cell = gb + 2 * ((size_t)kk * slice + pos);
-                    const cpx<T> gv = {(T)cell[0], (T)cell[1]};
-                    sk[kk] = cadd(sk[kk], cmul(tap, gv));
-                }
-            }
-        }
-        // the whole group takes part in the butterfly, samples that are off included
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            sk[k].re = group_sum(sk[k].re);
-            sk[k].im = group_sum(sk[k].im);
-        }
-        if (on) {
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                if (conj_out) sk[k] = conjg(sk[k]);
-                sk[k] = cmul(sk[k], cpx<T>{cs, -sn});
-                sk[k].re *= wt[k];
-                sk[k].im *= wt[k];
-            }
-            if constexpr (MODE == MODE_4J) {  // S = Pinv^H S Qinv
-                const size_t j1 = ((jb1 + f) * a.spw_count + s) * a.chan + c;
-                const size_t j2 = ((jb2 + f) * a.spw_count + s) * a.chan + c;
-                const cpx<T> *A = reinterpret_cast<const cpx<T> *>(a.jones_inv) + 4 * j1;
-                const cpx<T> *B = reinterpret_cast<const cpx<T> *>(a.jones_inv) + 4 * j2;
-                const cpx<T> a0 = conjg(A[0]), a1 = conjg(A[1]), a2 = conjg(A[2]),
-                             a3 = conjg(A[3]);
-                const cpx<T> t0 = cadd(cmul(a0, sk[0]), cmul(a2, sk[2]));
-                const cpx<T> t1 = cadd(cmul(a0, sk[1]), cmul(a2, sk[3]));
-                const cpx<T> t2 = cadd(cmul(a1, sk[0]), cmul(a3, sk[2]));
-                const cpx<T> t3 = cadd(cmul(a1, sk[1]), cmul(a3, sk[3]));
-                sk[0] = cadd(cmul(t0, B[0]), cmul(t1, B[2]));
-                sk[1] = cadd(cmul(t0, B[1]), cmul(t1, B[3]));
-                sk[2] = cadd(cmul(t2, B[0]), cmul(t3, B[2]));
-                sk[3] = cadd(cmul(t2, B[1]), cmul(t3, B[3]));
-            }
-#pragma unroll
-            for (int k = 0; k < NC; ++k) acc[k] = cadd(acc[k], sk[k]);
-        }
-    }
-    if (!in_range) return;
-    for (uint32_t cc = (uint32_t)gl; cc < a.npol; cc += GL) {
+template <int MODE, int PATH>
+__device__ __forceinline__ void store(const DArgs &d, const Sample<MODE, PATH> &sm,
+                                      const cpx<typename PathTraits<PATH>::acc_t> (&acc)[ModeTraits<MODE>::NCORR]) {
+    constexpr int NC = ModeTraits<MODE>::NCORR;
+    typedef typename PathTraits<PATH>::acc_t T;
+    if (!sm.in_range) return;
+    for (uint32_t cc = 0; cc < d.g.npol; ++cc) {
         cpx<T> val = {T(0), T(0)};
 #pragma unroll
         for (int k = 0; k < NC; ++k)
-            if (a.pol_idx[k] == cc) val = cadd(val, acc[k]);
-        d.out[2 * (base + cc)] = (visibility_base_type)val.re;
-        d.out[2 * (base + cc) + 1] = (visibility_base_type)val.im;
+            if (d.g.pol_idx[k] == cc) val = cadd(val, acc[k]);
+        d.out[2 * (sm.base + cc)] = (visibility_base_type)val.re;
+        d.out[2 * (sm.base + cc) + 1] = (visibility_base_type)val.im;
     }
 }
 
+__device__ __forceinline__ const grid_base_type *slice_of(const DArgs &d, uint32_t f, uint64_t cgi) {
+    return d.model + ((size_t)f * d.g.cube + cgi) * d.P * ((size_t)d.g.nx * d.g.ny) * 2;
+}
+
+// AA, W compile-time: a lane sums its sample's footprint.
+template <int MODE, int PATH, int W>
+__global__ __launch_bounds__(BLOCK) void degrid_aa_kernel(DArgs d) {
+    constexpr int NC = ModeTraits<MODE>::NCORR;
+    typedef typename PathTraits<PATH>::acc_t T;
+    const GridArgs &a = d.g;
+    extern __shared__ __align__(16) unsigned char smem[];
+    T *conv = reinterpret_cast<T *>(smem);
+    for (uint32_t i = threadIdx.x; i < a.csz; i += BLOCK)
+        conv[i] = reinterpret_cast<const T *>(a.conv)[i];
+    __syncthreads();
+    Sample<MODE, PATH> sm;
+    sm.load(d, (uint64_t)blockIdx.x * BLOCK + threadIdx.x);
+    const size_t slice = (size_t)a.nx * a.ny;
+    cpx<T> acc[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[k] = {T(0), T(0)};
+    for (uint32_t f = 0; f < a.facets; ++f) {
+        const Place<T> p = place<MODE, PATH, false>(d, sm, f);
+        if (!p.on) continue;
+        T cu[W];
+#pragma unroll
+        for (int k = 0; k < W; ++k) cu[k] = conv[p.fu + k * (int)a.OS];
+        const grid_base_type *g =
+            slice_of(d, f, sm.cgi) + 2 * ((size_t)p.y0 * a.nx + (size_t)p.x0);
+        cpx<T> sk[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) sk[k] = {T(0), T(0)};
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            const T cv = conv[p.fv + j * (int)a.OS];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                grid_base_type m[2 * W];   // a row of the footprint, in wide loads
+                __builtin_memcpy(m, g + 2 * ((size_t)c * slice + (size_t)j * a.nx), sizeof m);
+                cpx<T> t = {T(0), T(0)};
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    t.re = fma(cu[k], (T)m[2 * k], t.re);
+                    t.im = fma(cu[k], (T)m[2 * k + 1], t.im);
+                }
+                sk[c].re = fma(cv, t.re, sk[c].re);
+                sk[c].im = fma(cv, t.im, sk[c].im);
+            }
+        }
+        finish(d, sm, p, f, sk, acc);
+    }
+    store(d, sm, acc);
+}
+
+template <typename T> __device__ __forceinline__ T xor_lane(T v, int mask) {
+    return __shfl_xor(v, mask, 64);
+}
+
+// Any kernel: the wavefront sums the footprints of its 64 samples one after the other.
+template <int MODE, int PATH, bool WPROJ>
+__global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
+    constexpr int NC = ModeTraits<MODE>::NCORR;
+    typedef typename PathTraits<PATH>::acc_t T;
+    const GridArgs &a = d.g;
+    __shared__ cpx<T> res[BLOCK / 64][64][NC];
+    const int lane = threadIdx.x & 63;
+    cpx<T>(*mine)[NC] = res[threadIdx.x >> 6];
+    Sample<MODE, PATH> sm;
+    sm.load(d, (uint64_t)blockIdx.x * BLOCK + threadIdx.x);
+    const size_t slice = (size_t)a.nx * a.ny;
+    const T *conv = reinterpret_cast<const T *>(a.conv);
+    const cpx<T> *wtaps = reinterpret_cast<const cpx<T> *>(d.taps);
+    cpx<T> acc[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[k] = {T(0), T(0)};
+    for (uint32_t f = 0; f < a.facets; ++f) {
+        const Place<T> p = place<MODE, PATH, WPROJ>(d, sm, f);
+        const uint64_t on = __ballot(p.on);
+        for (int r0 = 0; r0 < 64; r0 += PACK) {
+            if (!((on >> r0) & ((1ull << PACK) - 1))) continue;
+            cpx<T> part[PACK][NC];
+#pragma unroll
+            for (int j = 0; j < PACK; ++j) {
+#pragma unroll
+                for (int k = 0; k < NC; ++k) part[j][k] = {T(0), T(0)};
+                const int r = r0 + j;
+                if (!((on >> r) & 1)) continue;
+                // the sample's place, in scalar registers
+                const uint32_t wp = (uint32_t)__builtin_amdgcn_readlane(p.wp, r);
+                const uint32_t tb = (uint32_t)__builtin_amdgcn_readlane((int)p.tb, r);
+                const int x0 = __builtin_amdgcn_readlane(p.x0, r);
+                const int y0 = __builtin_amdgcn_readlane(p.y0, r);
+                const int fu = __builtin_amdgcn_readlane(p.fu, r);
+                const int fv = __builtin_amdgcn_readlane(p.fv, r);
+                const uint32_t cg = (uint32_t)__builtin_amdgcn_readlane((int)sm.cgi, r);
+                const grid_base_type *g = slice_of(d, f, cg) + 2 * ((size_t)y0 * a.nx + (size_t)x0);
+                // t / wp for t < 64^2: t * (2^20 / wp + 1) >> 20 is exact (t times the
+                // reciprocal's excess stays below 2^20)
+                const uint32_t inv = (1u << 20) / wp + 1;
+                const uint32_t ntap = wp * wp;
+                for (uint32_t t = (uint32_t)lane; t < ntap; t += 64) {
+                    const uint32_t y = (t * inv) >> 20, x = t - y * wp;
+                    cpx<T> tap;   // conjugated
+                    if constexpr (WPROJ) {
+                        const cpx<T> tw = wtaps[tb + t];
+                        tap = {tw.re, -tw.im};
+                    } else {
+                        tap = {conv[fu + x * a.OS] * conv[fv + y * a.OS], T(0)};
+                    }
+                    const grid_base_type *cell = g + 2 * ((size_t)y * a.nx + x);
+#pragma unroll
+                    for (int k = 0; k < NC; ++k) {
+                        const cpx<T> gv = {(T)cell[2 * (size_t)k * slice],
+                                           (T)cell[2 * (size_t)k * slice + 1]};
+                        part[j][k] = cmac(part[j][k], tap, gv);
+                    }
+                }
+            }
+            // reduce: at each of three steps a lane keeps the half of the samples that its bit
+            // names and adds its partner's sums for them; then three plain steps
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                cpx<T> v[PACK];
+#pragma unroll
+                for (int j = 0; j < PACK; ++j) v[j] = part[j][k];
+#pragma unroll
+                for (int h = PACK / 2, m = 32; h >= 1; h /= 2, m /= 2) {
+                    const bool up = (lane & m) != 0;
+#pragma unroll
+                    for (int j = 0; j < h; ++j) {
+                        const cpx<T> keep = up ? v[j + h] : v[j], give = up ? v[j] : v[j + h];
+                        v[j].re = keep.re + xor_lane(give.re, m);
+                        v[j].im = keep.im + xor_lane(give.im, m);
+                    }
+                }
+#pragma unroll
+                for (int m = 64 / PACK / 2; m >= 1; m /= 2) {
+                    v[0].re += xor_lane(v[0].re, m);
+                    v[0].im += xor_lane(v[0].im, m);
+                }
+                if ((lane & (64 / PACK - 1)) == 0) mine[r0 + lane / (64 / PACK)][k] = v[0];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (p.on) {
+            cpx<T> sk[NC];
+#pragma unroll
+            for (int k = 0; k < NC; ++k) sk[k] = mine[lane][k];
+            finish(d, sm, p, f, sk, acc);
+        }
+    }
+    store(d, sm, acc);
+}
+
 template <int MODE, int PATH> static hipError_t launch_t(const DArgs &d, hipStream_t st) {
-    const uint64_t threads = d.rows * d.g.chan * GL;
-    const uint64_t blocks = (threads + BLOCK - 1) / BLOCK;
+    const uint64_t blocks = (d.rows * d.g.chan + BLOCK - 1) / BLOCK;
     if (!blocks) return hipSuccess;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    degrid_kernel<MODE, PATH><<<dim3((uint32_t)blocks), dim3(BLOCK), 0, st>>>(d);
+    const dim3 g((uint32_t)blocks), b(BLOCK);
+    const size_t smem = (size_t)d.g.csz * sizeof(typename PathTraits<PATH>::acc_t);
+    if (d.wproj)
+        degrid_wave_kernel<MODE, PATH, true><<<g, b, 0, st>>>(d);
+    else if (smem > 32768)   // an oversampling far beyond use: the taps stay in memory
+        degrid_wave_kernel<MODE, PATH, false><<<g, b, 0, st>>>(d);
+    else
+        switch (d.g.W) {
+            case 3: degrid_aa_kernel<MODE, PATH, 3><<<g, b, smem, st>>>(d); break;
+            case 5: degrid_aa_kernel<MODE, PATH, 5><<<g, b, smem, st>>>(d); break;
+            case 7: degrid_aa_kernel<MODE, PATH, 7><<<g, b, smem, st>>>(d); break;
+            case 9: degrid_aa_kernel<MODE, PATH, 9><<<g, b, smem, st>>>(d); break;
+            case 11: degrid_aa_kernel<MODE, PATH, 11><<<g, b, smem, st>>>(d); break;
+            default: degrid_wave_kernel<MODE, PATH, false><<<g, b, 0, st>>>(d);
+        }
     return hipGetLastError();
 }
 
