@@ -27,6 +27,7 @@
 #include <chrono>
 
 #include "host_common.h"
+#include "wtile.h"
 
 namespace bam {
 
@@ -72,8 +73,22 @@ struct Launch {
     bool single;         // one facet's launch of the single-facet kernels
 };
 
+// One pass of the tiled gridder (wtile.hip) over facets of one kind and a range of rows.
+struct TilePass {
+    wt::TArgs t;
+    wt::Plan plan;
+    int kind;
+};
+
 struct Plan {
     bool ready = false;
+    // Default tiles: the tiled gridder, with its facet lists and first spots (tile_ints, per pass),
+    // the channel table of each kind and the workspace the passes take turns in.
+    bool tiled = false;
+    std::vector<TilePass> passes;
+    std::vector<uint32_t> tile_ints_host;
+    uint8_t widths[32] = {};
+    DevBuf tile_ints, tile_ws, chan_vis, chan_psf;
     int mode = MODE_1, schedule = 0, path = PATH_F32K;
     uint32_t n = 0, NC = 1, cube = 1, sfC = 1, cubeB = 1;
     uint32_t B = 0, C = 0, cps = 1, ncb = 1, base_rows = 32, nseg_base = 1, rows = 0;
@@ -101,6 +116,9 @@ struct Plan {
     hipStream_t side[BRANCHES - 1] = {};
     hipEvent_t fork = nullptr, join[BRANCHES - 1] = {}, t0 = nullptr, t1 = nullptr;
 
+    const uint64_t *cgi_vis = nullptr, *cgi_psf = nullptr;
+    const uint64_t *cgi_of(int kind) const { return kind == MODE_PSF ? cgi_psf : cgi_vis; }
+
     void drop_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
@@ -109,7 +127,7 @@ struct Plan {
     }
     void release() {
         drop_graph();
-        DevBuf *bufs[] = {&acc, &norm, &fargs, &geom, &lists, &lists64, &queues, &cls_all,
+        DevBuf *bufs[] = {&tile_ints, &tile_ws, &chan_vis, &chan_psf, &acc, &norm, &fargs, &geom, &lists, &lists64, &queues, &cls_all,
                           &out_tmp, &walk,
                           &in_vis, &in_uvw, &in_w, &in_flags, &in_rowflags, &in_field, &in_spw,
                           &in_a1, &in_a2, &in_wl, &in_enabled, &in_cgi, &in_sfcgi, &perm, &rowrec, &keys,
@@ -126,6 +144,7 @@ struct Plan {
         if (t1) (void)hipEventDestroy(t1);
         fork = t0 = t1 = nullptr;
         launches.clear();
+        passes.clear();
         lists_host.clear();
         lists_host.shrink_to_fit();
         lists64_host.clear();
@@ -433,9 +452,26 @@ hipError_t issue(const Plan &pl, const Launch &L, int shape, hipStream_t st) {
 int enqueue_all(Plan &pl, hipStream_t st) {
     // the row table is gathered from the row arrays on every pass: with device-resident buffers
     // the caller's arrays are read in place, so changes after planning are seen
-    HIP_TRY(build_row_tables(pl.base, pl.rows, false, pl.rowrec.as<RowRec>(), nullptr, st));
+    HIP_TRY(build_row_tables(pl.base, pl.rows, false, pl.rowrec.as<RowRec>(), nullptr, st,
+                             pl.tiled));
     HIP_TRY(fill_f64(pl.acc.as<double>(), pl.acc_elems, 0.0, st));
     HIP_TRY(fill_f64(pl.norm.as<double>(), pl.norm_stride * pl.base.nslots, 0.0, st));
+    if (pl.tiled) {
+        for (int kind : {pl.mode, (int)MODE_PSF}) {
+            GridArgs a = pl.base;
+            const TilePass *first = nullptr;
+            for (const TilePass &q : pl.passes)
+                if (q.kind == kind && !first) first = &q;
+            if (!first) continue;
+            a.cgi = pl.cgi_of(kind);
+            HIP_TRY(build_row_tables(a, 0, false, nullptr,
+                                     const_cast<ChanRec *>(first->t.w.g.chanrec), st));
+        }
+        for (const TilePass &q : pl.passes)
+            HIP_TRY(wtile_grid(q.t, q.plan, pl.tile_ws.p, q.kind, pl.path == PATH_FP64, pl.widths,
+                               st, pl.side, BRANCHES - 1, pl.fork, pl.join));
+        return 0;
+    }
     if (pl.schedule != BULLSEYE_BATCH_PER_FACET)
         HIP_TRY(fill_u32(pl.queues.as<uint32_t>(), (uint32_t)pl.launches.size(), 0u, st));
     bool used[BRANCHES] = {false, false, false, false};
@@ -471,9 +507,108 @@ int capture(Plan &pl, hipStream_t st) {
     return 0;
 }
 
+// The passes of the tiled gridder: facets of one kind together while their samples' records stay
+// within 4 GiB (halved while the workspace cannot be had), rows split where one facet's do not.
+// pl.tiled stays false where a facet's bins cannot be numbered.
+int plan_tiles(Plan &pl) {
+    const LibView lv = lib_view();
+    const bool fp64 = pl.path == PATH_FP64;
+    pl.passes.clear();
+    pl.tile_ints_host.clear();
+    uint32_t lo = 31, hi = 0;
+    memset(pl.widths, 0, sizeof pl.widths);
+    for (uint32_t f = 0; f < pl.n; ++f)
+        for (uint32_t h : sets[pl.fset[f]].half) {
+            pl.widths[h] = 1;
+            lo = std::min(lo, h);
+            hi = std::max(hi, h);
+        }
+    const size_t nfc = (size_t)pl.base.spw_count * pl.C;
+    HIP_TRY(pl.chan_vis.ensure(std::max<size_t>(1, nfc) * sizeof(ChanRec)));
+    HIP_TRY(pl.chan_psf.ensure(std::max<size_t>(1, nfc) * sizeof(ChanRec)));
+    const uint64_t per_row = pl.C;
+    for (uint64_t bytes = (uint64_t)4 << 30;; bytes /= 2) {
+        pl.passes.clear();
+        pl.tile_ints_host.clear();
+        size_t ws = 0;
+        for (int kind : {pl.mode, (int)MODE_PSF}) {
+            const uint32_t nc = kind == MODE_PSF ? 1 : pl.NC;
+            const uint64_t cap = bytes / (sizeof(wt::Head) + 4 + (size_t)nc * (fp64 ? 16 : 8));
+            const uint64_t rows1 = std::max<uint64_t>(
+                1, std::min<uint64_t>(pl.rows, cap / std::max<uint64_t>(1, per_row)));
+            const uint64_t samples1 = std::max<uint64_t>(1, rows1 * per_row);
+            uint32_t f = 0;
+            while (f < pl.n) {
+                // the next facets of this kind that fit one pass
+                const size_t at = pl.tile_ints_host.size();
+                std::vector<uint32_t> list, base;
+                uint64_t spots = 0;
+                wt::Plan wp{};
+                for (; f < pl.n; ++f) {
+                    if (pl.fkind[f] != kind) continue;
+                    const uint64_t more = (uint64_t)pl.fcube[f] * wt::tiles_of(pl.facets[f].nx) *
+                                          wt::tiles_of(pl.facets[f].ny);
+                    wt::Plan next;
+                    const uint64_t total = samples1 * (list.size() + 1);
+                    if ((!list.empty() && (total > cap || list.size() >= 65535)) ||
+                        !wtile_plan(next, total, spots + more, lo, hi, (int)nc, fp64)) {
+                        if (list.empty()) return 0;   // the class lists take this batch
+                        break;
+                    }
+                    wp = next;
+                    list.push_back(f);
+                    base.push_back((uint32_t)spots);
+                    spots += more;
+                }
+                if (list.empty()) break;
+                ws = std::max(ws, wp.total);
+                pl.tile_ints_host.insert(pl.tile_ints_host.end(), list.begin(), list.end());
+                pl.tile_ints_host.insert(pl.tile_ints_host.end(), base.begin(), base.end());
+                for (uint64_t r0 = 0; r0 < pl.rows; r0 += rows1) {
+                    TilePass q;
+                    memset(&q.t, 0, sizeof q.t);
+                    q.kind = kind;
+                    q.plan = wp;   // (a shorter last range of rows fits the full range's plan)
+                    q.t.w.g = pl.base;
+                    q.t.w.g.cube = pl.cubeB;
+                    q.t.w.g.chanrec =
+                        kind == MODE_PSF ? pl.chan_psf.as<ChanRec>() : pl.chan_vis.as<ChanRec>();
+                    q.t.nfacets = (uint32_t)list.size();
+                    q.t.row0 = (uint32_t)r0;
+                    q.t.row1 = (uint32_t)std::min<uint64_t>(pl.rows, r0 + rows1);
+                    // offsets until the upload
+                    q.t.facet_list = (const uint32_t *)(uintptr_t)at;
+                    q.t.spot_base = (const uint32_t *)(uintptr_t)(at + list.size());
+                    pl.passes.push_back(q);
+                }
+            }
+        }
+        const hipError_t e = pl.tile_ws.ensure(std::max<size_t>(ws, 16));
+        if (e == hipErrorOutOfMemory && bytes > ((uint64_t)16 << 20)) {
+            (void)hipGetLastError();
+            continue;
+        }
+        HIP_TRY(e);
+        break;
+    }
+    HIP_TRY(pl.tile_ints.ensure(std::max<size_t>(4, pl.tile_ints_host.size() * 4)));
+    if (!pl.tile_ints_host.empty())
+        HIP_TRY(hipMemcpyAsync(pl.tile_ints.p, pl.tile_ints_host.data(),
+                               pl.tile_ints_host.size() * 4, hipMemcpyHostToDevice, lv.stream));
+    HIP_TRY(hipStreamSynchronize(lv.stream));
+    for (TilePass &q : pl.passes) {
+        q.t.w.facet_args = pl.fargs.as<wp::WArgs>();
+        q.t.facet_list = pl.tile_ints.as<uint32_t>() + (uintptr_t)q.t.facet_list;
+        q.t.spot_base = pl.tile_ints.as<uint32_t>() + (uintptr_t)q.t.spot_base;
+    }
+    pl.tiled = true;
+    return 0;
+}
+
 // Everything of a plan up to the lists: staging, sort, geometry, facet table, classes.
+// tiled: plan the tiled gridder, else (or where its bins cannot be numbered) the class lists.
 int build_plan(gridding_parameters *p, int mode, const bullseye_batch_facet *facets, uint32_t n,
-               int schedule, const bullseye_batch_tuning &t, Plan &pl) {
+               int schedule, const bullseye_batch_tuning &t, Plan &pl, bool tiled) {
     const LibView lv = lib_view();
     if (validate(lv, p, mode, facets, n)) return 1;
     if (schedule < 0 || schedule > BULLSEYE_BATCH_PER_FACET) return fail("unknown batch schedule");
@@ -531,6 +666,8 @@ int build_plan(gridding_parameters *p, int mode, const bullseye_batch_facet *fac
                   nspw * C * sizeof(size_t), &d));
     const uint64_t *cgi_psf = (const uint64_t *)d;
     a.cgi = cgi_vis ? cgi_vis : cgi_psf;
+    pl.cgi_vis = cgi_vis;
+    pl.cgi_psf = cgi_psf;
 
     // ingest: stable sort of rows by baseline
     HIP_TRY(pl.perm.ensure(rows * 4));
@@ -699,6 +836,9 @@ int build_plan(gridding_parameters *p, int mode, const bullseye_batch_facet *fac
         w.nf = ks.nf;
         w.fbase = ks.fbase;
         w.wmax_f = ks.wmax;
+        w.inv_wmax = 1.0 / (double)ks.wmax;
+        w.base_rows = pl.base_rows;
+        w.nseg_base = pl.nseg_base;
         w.seg_cls = pl.cls_all.as<uint8_t>() + (size_t)pl.set_slot[fc.kernel_set] * pl.nbase;
     }
     HIP_TRY(pl.fargs.ensure(n * sizeof(wp::WArgs)));
@@ -715,12 +855,23 @@ int build_plan(gridding_parameters *p, int mode, const bullseye_batch_facet *fac
             HIP_TRY(hipEventCreateWithFlags(&pl.join[b], hipEventDisableTiming));
         }
     }
-    return build_lists(pl, t);
+    pl.tiled = false;
+    if (tiled && plan_tiles(pl)) return 1;
+    return pl.tiled ? 0 : build_lists(pl, t);
+}
+
+// Whether the tuning leaves the tiles at their default: the tiled gridder.
+bool default_tiles(const bullseye_batch_tuning &t) {
+    for (uint32_t i = 0; i < NCLS; ++i)
+        if (t.shape[i] != WSHAPE_DEFAULT || t.chunk[i] > 1) return false;
+    return !t.facet_major;
 }
 
 int plan_impl(gridding_parameters *p, int mode, const bullseye_batch_facet *facets, uint32_t n,
               int schedule) {
-    if (build_plan(p, mode, facets, n, schedule, tuning, plan)) return 1;
+    if (build_plan(p, mode, facets, n, schedule, tuning, plan,
+                   schedule != BULLSEYE_BATCH_PER_FACET && default_tiles(tuning)))
+        return 1;
     if (schedule == BULLSEYE_BATCH_PERSISTENT_GRAPH && capture(plan, lib_view().stream)) return 1;
     plan.ready = true;
     return 0;
@@ -852,7 +1003,8 @@ int autotune_impl(gridding_parameters *p, int mode, const bullseye_batch_facet *
                 t.channels_per_stream = cps;
                 t.base_rows = base;
                 for (uint32_t i = 0; i < NCLS; ++i) t.chunk[i] = chunk;
-                if (build_plan(p, mode, facets, n, BULLSEYE_BATCH_PERSISTENT, t, plan)) return 1;
+                if (build_plan(p, mode, facets, n, BULLSEYE_BATCH_PERSISTENT, t, plan, false))
+                    return 1;
                 double ms_cls[4][NCLS];
                 for (auto &row : ms_cls)
                     for (double &v : row) v = 0;
@@ -911,7 +1063,7 @@ int autotune_impl(gridding_parameters *p, int mode, const bullseye_batch_facet *
     for (uint32_t fm = 0; fm < 2; ++fm) {
         bullseye_batch_tuning t = best_t;
         t.facet_major = fm;
-        if (build_plan(p, mode, facets, n, BULLSEYE_BATCH_PERSISTENT, t, plan)) return 1;
+        if (build_plan(p, mode, facets, n, BULLSEYE_BATCH_PERSISTENT, t, plan, false)) return 1;
         for (size_t j = 0; j < plan.launches.size(); ++j) {
             double ms = 0;
             if (time_launch(plan, j, plan.launches[j].shape, ms)) return 1;
@@ -921,6 +1073,31 @@ int autotune_impl(gridding_parameters *p, int mode, const bullseye_batch_facet *
     if (check_device_errors()) return 1;
     best_t.facet_major = order_ms[1] < order_ms[0] ? 1 : 0;
     best_total = std::min(order_ms[0], order_ms[1]);
+    // the tiled gridder, which the default tiles stand for, against the tuned class kernels
+    {
+        bullseye_batch_tuning t = best_t;
+        for (uint32_t i = 0; i < NCLS; ++i) t.shape[i] = t.chunk[i] = 0;
+        t.facet_major = 0;
+        if (build_plan(p, mode, facets, n, BULLSEYE_BATCH_PERSISTENT, t, plan, true)) return 1;
+        if (plan.tiled) {
+            double best = 1e300;
+            for (int rep = 0; rep < 2; ++rep) {
+                HIP_TRY(hipEventRecord(plan.t0, lv.stream));
+                if (enqueue_all(plan, lv.stream)) return 1;
+                HIP_TRY(hipEventRecord(plan.t1, lv.stream));
+                HIP_TRY(hipStreamSynchronize(lv.stream));
+                float ms = 0;
+                HIP_TRY(hipEventElapsedTime(&ms, plan.t0, plan.t1));
+                best = std::min(best, (double)ms);
+            }
+            if (check_device_errors()) return 1;
+            default_total = best;
+            if (best <= best_total) {
+                best_t = t;
+                best_total = best;
+            }
+        }
+    }
     plan.release();
     best_t.tuned = 1;
     best_t.tuned_ms = best_total;

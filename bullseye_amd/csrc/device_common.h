@@ -45,7 +45,7 @@ struct __align__(16) RowRec {
     uint32_t row;          // original row index (visibility, weight and flag addressing)
     uint32_t spw;          // spectral window as given (range-checked by the kernel)
     uint32_t state;        // ROW_* bits
-    uint32_t pad;
+    uint32_t bl;           // baseline (batches only)
     uint64_t j1, j2;       // Jones modes: (t * antennas + ant) * facets * spw_count * chan
 };
 

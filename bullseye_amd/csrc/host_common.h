@@ -64,8 +64,9 @@ hipError_t finalize_device(void *buf, uint32_t F, uint32_t n, uint32_t fstride, 
                            uint32_t ny, const double *tx, const double *ty, void *scratch,
                            bool place_real, hipStream_t st);
 hipError_t fill_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t st);
+// rowrec, chanrec: nullptr leaves that table out; baselines: fill RowRec::bl
 hipError_t build_row_tables(const GridArgs &a, uint32_t rows, bool jones, RowRec *rowrec,
-                            ChanRec *chanrec, hipStream_t st);
+                            ChanRec *chanrec, hipStream_t st, bool baselines = false);
 hipError_t launch_facet_geom(const uvw_base_type *fc, double ra0, double dec0, uint32_t F,
                              bool facet, bool phase, FacetGeom *out, hipStream_t st);
 

@@ -175,7 +175,8 @@ __global__ void k_walk_decide(const double *part, int override_order, int *time_
 // (t * antennas + ant) * facets * spw_count * chan; the gridding kernel raises the error for a
 // row with bad ids when one of its samples reaches the Jones correction, as it would have
 // reading the ids itself.
-__global__ void k_row_table(GridArgs a, uint32_t rows, int jones, uint64_t fsc, RowRec *out) {
+__global__ void k_row_table(GridArgs a, uint32_t rows, int jones, int baselines, uint64_t fsc,
+                            RowRec *out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= rows) return;
     const uint32_t row = a.perm[i];
@@ -186,7 +187,17 @@ __global__ void k_row_table(GridArgs a, uint32_t rows, int jones, uint64_t fsc, 
     r.row = row;
     r.spw = a.spw[row];
     r.state = (!a.row_flags[row] && a.field[row] == a.imaging_field) ? ROW_USABLE : 0u;
-    r.pad = 0;
+    r.bl = 0;
+    if (baselines) {   // the last baseline that starts at or before sorted row i
+        uint32_t hi = a.baselines;
+        while (hi - r.bl > 1) {
+            const uint32_t mid = (r.bl + hi) / 2;
+            if (a.bl_start[mid] <= i)
+                r.bl = mid;
+            else
+                hi = mid;
+        }
+    }
     r.j1 = r.j2 = 0;
     if (jones) {
         const uint64_t t = a.time_ids[row];
@@ -213,12 +224,13 @@ __global__ void k_chan_table(GridArgs a, uint32_t n, ChanRec *out) {
 }
 
 hipError_t build_row_tables(const GridArgs &a, uint32_t rows, bool jones, RowRec *rowrec,
-                            ChanRec *chanrec, hipStream_t st) {
+                            ChanRec *chanrec, hipStream_t st, bool baselines) {
     const uint32_t nfc = a.spw_count * a.chan;
     if (nfc && chanrec) k_chan_table<<<(nfc + 255) / 256, 256, 0, st>>>(a, nfc, chanrec);
-    if (rows) {
+    if (rows && rowrec) {
         const uint64_t fsc = (uint64_t)a.facets * a.spw_count * a.chan;
-        k_row_table<<<(rows + 255) / 256, 256, 0, st>>>(a, rows, jones ? 1 : 0, fsc, rowrec);
+        k_row_table<<<(rows + 255) / 256, 256, 0, st>>>(a, rows, jones ? 1 : 0,
+                                                          baselines ? 1 : 0, fsc, rowrec);
     }
     return hipGetLastError();
 }

@@ -25,6 +25,7 @@ struct Item {        // up to TArgs::chunk consecutive records of one bin
 struct TArgs {
     wp::WArgs w;                 // call arguments; w.facet_args: per-facet arguments of a batch
     uint32_t f0, nfacets;        // facets of this pass
+    const uint32_t *facet_list;  // batch: the pass's facets
     uint32_t row0, row1;         // sorted rows of this pass
     const uint32_t *spot_base;   // batch: first spot (slice, tile) of each facet of the pass
     uint32_t nspots;             // spots of the pass's facets
@@ -52,10 +53,10 @@ struct Plan {
 // exceed what one pass can number.
 bool wtile_plan(wt::Plan &p, uint64_t samples, uint64_t spots, uint32_t half_lo, uint32_t half_hi,
                 int ncorr, bool fp64);
-// One pass: t.w, facets, rows and spot_base set by the caller, the rest from the plan's
+// One pass: t.w, facets, rows and (batch) facet_list and spot_base set by the caller, the rest from the plan's
 // workspace.  widths[h] != 0: some plane has half support h.  The width launches are dealt over
 // st and the side streams, forked and joined by events.
-hipError_t wtile_grid(wt::TArgs t, const wt::Plan &p, void *ws, int mode, bool fp64,
+hipError_t wtile_grid(const wt::TArgs &t, const wt::Plan &p, void *ws, int mode, bool fp64,
                       const uint8_t *widths, hipStream_t st, hipStream_t *side, int nside,
                       hipEvent_t fork, hipEvent_t *join);
 

@@ -91,12 +91,13 @@ __device__ __forceinline__ bool locate(const wp::WArgs &w, const FacetGeom *gp, 
 }
 
 // One (sorted row, channel) of a facet: the checks of the class kernels in their order, the
-// weights, and the position.  Errors are raised only in the scattering pass.
-template <int MODE, bool RAISE>
-__device__ __forceinline__ bool find(const wp::WArgs &w, const FacetGeom *gp, uint32_t ri,
-                                     uint32_t c, RowRec &rr, uint32_t &cgi, double &u, double &v,
-                                     double &ww, size_t &base, Spot &s) {
-    const GridArgs &a = w.g;
+// weights, and the position.  Errors are raised only in the scattering pass.  The arrays shared by
+// the facets come from the launch's arguments (t.w.g), the facet's own from w.
+template <int MODE, bool RAISE, bool BATCH>
+__device__ __forceinline__ bool find(const TArgs &t, const wp::WArgs &w, const FacetGeom *gp,
+                                     uint32_t ri, uint32_t c, RowRec &rr, uint32_t &cgi, double &u,
+                                     double &v, double &ww, size_t &base, Spot &s) {
+    const GridArgs &a = t.w.g;
     rr = load_row_record(a.rowrec + ri);
     if (rr.spw >= a.spw_count) {
         if (RAISE) atomicOr(a.error_flag, 4);
@@ -104,7 +105,7 @@ __device__ __forceinline__ bool find(const wp::WArgs &w, const FacetGeom *gp, ui
     }
     const ChanRec ch = a.chanrec[rr.spw * a.chan + c];
     if (!ch.enabled) return false;
-    if (ch.cgi >= a.cube) {
+    if (ch.cgi >= w.g.cube) {
         if (RAISE) atomicOr(a.error_flag, 4);
         return false;
     }
@@ -129,10 +130,22 @@ __device__ __forceinline__ bool find(const wp::WArgs &w, const FacetGeom *gp, ui
         }
         if (!any) return false;
     }
-    return locate(w, gp, u, v, ww, s);
+    if (!locate(w, gp, u, v, ww, s)) return false;
+    if constexpr (BATCH) {
+        // a plan is of the data it was made from: a sample wider than the class its stream had
+        // then is dropped and reported, as the class kernels do
+        const uint32_t seg = (ri - a.bl_start[rr.bl]) / w.base_rows;
+        const uint64_t entry =
+            ((uint64_t)rr.bl * a.n_chan_blocks + c / a.chan_per_stream) * w.nseg_base + seg;
+        if (2 * s.half + 1 > (int)w.seg_cls[entry]) {
+            if (RAISE) atomicOr(a.error_flag, 8);
+            return false;
+        }
+    }
+    return true;
 }
 
-// Bin of a located sample: widths, then slices of the facets, then tiles.
+// Bin of a located sample of the pass's facet f: widths, then slices of the facets, then tiles.
 __device__ __forceinline__ uint32_t bin_of(const TArgs &t, const wp::WArgs &w, uint32_t f,
                                            uint32_t cgi, const Spot &s) {
     const uint32_t tx = (uint32_t)s.x0 / TILE, ty = (uint32_t)s.y0 / TILE;
@@ -194,14 +207,14 @@ struct Walk {
 constexpr uint32_t NO_BIN = 0xffffffffu;
 
 template <int MODE, bool BATCH> __global__ __launch_bounds__(BLOCK) void k_count(TArgs t) {
-    const uint32_t f = t.f0 + blockIdx.y;
+    const uint32_t f = BATCH ? t.facet_list[blockIdx.y] : t.f0 + blockIdx.y;
     const wp::WArgs &w = BATCH ? t.w.facet_args[f] : t.w;
     const FacetGeom *gp = w.g.geom + (BATCH ? 0 : f);
     const uint32_t lane = threadIdx.x & 63, copy = blockIdx.x % t.copies;
     const uint32_t wave = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
     uint32_t run = NO_BIN, run_n = 0, run_at = 0;
-    Walk k(wave * 64 * t.iters + lane, t.row0, w.g.chan,
-           blockIdx.y * (t.row1 - t.row0) * w.g.chan);
+    Walk k(wave * 64 * t.iters + lane, t.row0, t.w.g.chan,
+           blockIdx.y * (t.row1 - t.row0) * t.w.g.chan);
     for (uint32_t it = 0; it < t.iters; ++it, k.next()) {
         RowRec rr;
         uint32_t cgi, bin = 0;
@@ -209,8 +222,8 @@ template <int MODE, bool BATCH> __global__ __launch_bounds__(BLOCK) void k_count
         size_t base;
         Spot s;
         const bool live = k.row < t.row1 &&
-                          find<MODE, false>(w, gp, k.row, k.chan, rr, cgi, u, v, ww, base, s);
-        if (live) bin = bin_of(t, w, f - t.f0, cgi, s);
+                          find<MODE, false, BATCH>(t, w, gp, k.row, k.chan, rr, cgi, u, v, ww, base, s);
+        if (live) bin = bin_of(t, w, blockIdx.y, cgi, s);
         const uint64_t any = __ballot(live);
         if (!any) continue;
         const int lead = __ffsll((unsigned long long)any) - 1;
@@ -241,10 +254,11 @@ template <int MODE, bool BATCH> __global__ __launch_bounds__(BLOCK) void k_count
 template <int MODE, typename T, bool BATCH>
 __global__ __launch_bounds__(BLOCK) void k_scatter(TArgs t) {
     constexpr int NC = ModeTraits<MODE>::NCORR;
-    const uint32_t f = t.f0 + blockIdx.y;
+    const uint32_t f = BATCH ? t.facet_list[blockIdx.y] : t.f0 + blockIdx.y;
     const wp::WArgs &w = BATCH ? t.w.facet_args[f] : t.w;
     const FacetGeom *gp = w.g.geom + (BATCH ? 0 : f);
-    const GridArgs &a = w.g;
+    const GridArgs &a = t.w.g;
+    const bool phase = w.g.phase != 0;
     const uint32_t lane = threadIdx.x & 63, copy = blockIdx.x % t.copies;
     const uint32_t wave = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
     struct __align__(sizeof(T) == 4 && NC == 1 ? 16 : 8) Rec {
@@ -268,10 +282,10 @@ __global__ __launch_bounds__(BLOCK) void k_scatter(TArgs t) {
         size_t base = 0;
         Spot s;
         const bool live = k.row < t.row1 &&
-                          find<MODE, true>(w, gp, k.row, k.chan, rr, cgi, u, v, ww, base, s);
+                          find<MODE, true, BATCH>(t, w, gp, k.row, k.chan, rr, cgi, u, v, ww, base, s);
         cpx<T> vis[NC];
         if (live) {
-            bin = bin_of(t, w, f - t.f0, cgi, s);
+            bin = bin_of(t, w, blockIdx.y, cgi, s);
             T wt[NC];
             if constexpr (MODE == MODE_PSF) {
                 vis[0] = {T(1), T(0)};
@@ -298,13 +312,13 @@ __global__ __launch_bounds__(BLOCK) void k_scatter(TArgs t) {
                 vis[3] = cmac(cmul(P[2], t1), P[3], t3);
             }
             T sn = T(0), cs = T(1);
-            if (a.phase) {   // phase_transform_policies.h:138-146, argument in turns, FP64
+            if (phase) {   // phase_transform_policies.h:138-146, argument in turns, FP64
                 const double turns = u * gp->dl + v * gp->dm + ww * gp->dn;
                 const double fr = 2.0 * (turns - rint(turns));
                 if constexpr (sizeof(T) == 8) {
                     sincospi(fr, &sn, &cs);
                 } else {
-                    sincospif((float)fr, &sn, &cs);
+                    sincospi_unit((float)fr, &sn, &cs);
                 }
             }
             const double ts = w.plane_norm[(size_t)s.plane * w.nf * w.nf + s.q];
@@ -318,7 +332,7 @@ __global__ __launch_bounds__(BLOCK) void k_scatter(TArgs t) {
             for (int c = 0; c < NC; ++c) {
                 vis[c].re *= wt[c];
                 vis[c].im *= wt[c];
-                if (a.phase) vis[c] = cmul(vis[c], cpx<T>{cs, sn});
+                if (phase) vis[c] = cmul(vis[c], cpx<T>{cs, sn});
                 if (s.neg) vis[c].im = -vis[c].im;
                 nacc[c] += (double)wt[c] * ts;
             }
@@ -414,14 +428,14 @@ __global__ __launch_bounds__(BLOCK) void k_items(TArgs t) {
         }
         in -= t.spot_base[f];
     }
-    const wp::WArgs &w = t.w.facet_args ? t.w.facet_args[t.f0 + f] : t.w;
+    const wp::WArgs &w = t.spot_base ? t.w.facet_args[t.facet_list[f]] : t.w;
     const uint32_t nx = tiles_of(w.g.nx), ny = tiles_of(w.g.ny);
     if (!t.spot_base) {
         f = in / (w.g.cube * nx * ny);
         in -= f * w.g.cube * nx * ny;
     }
     Item it;
-    it.facet = t.f0 + f;
+    it.facet = t.spot_base ? t.facet_list[f] : t.f0 + f;
     it.slice = in / (nx * ny);
     in -= it.slice * nx * ny;
     it.ty = (uint16_t)(in / nx);
@@ -460,6 +474,29 @@ template <> __device__ __forceinline__ double lane_value(double v, int l) {
                             __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
+// Taps in the global address space: a batch's pointers come from memory, and loads whose address
+// space the compiler cannot see wait for the LDS adds in flight as well.
+template <typename T> struct Taps {
+    typedef T v2 __attribute__((ext_vector_type(2)));
+    typedef const v2 __attribute__((address_space(1))) * ptr;
+    ptr p;
+    __device__ __forceinline__ explicit Taps(const void *q) : p((ptr)(uintptr_t)q) {}
+    __device__ __forceinline__ cpx<T> operator[](uint32_t i) const {
+        const v2 x = p[i];
+        return {x.x, x.y};
+    }
+    __device__ __forceinline__ Taps at(uint32_t i) const {
+        Taps t(*this);
+        t.p += i;
+        return t;
+    }
+};
+
+__device__ __forceinline__ void grid_add(double *p, double v) {
+    typedef __attribute__((address_space(1))) double gdouble;
+    (void)__builtin_amdgcn_global_atomic_fadd_f64((gdouble *)(uintptr_t)p, v);
+}
+
 // One tap of a sample: the product in the path's precision, added in FP64.
 template <int CELLS, typename T>
 __device__ __forceinline__ void add_tap(double *tile, uint32_t at, cpx<T> v, cpx<T> tap) {
@@ -484,7 +521,7 @@ __device__ __forceinline__ void add_item(const TArgs &t, const wp::WArgs &w, con
     constexpr int KU = K < 8 ? K : 8;                      // of them in flight together
     constexpr int U = PACK > 1 ? 2 : K == 1 ? 8 : K == 2 ? 4 : K < 4 ? 2 : 1;   // samples in flight
     const int lane = threadIdx.x & 63;
-    const cpx<T> *taps = reinterpret_cast<const cpx<T> *>(w.taps);
+    const Taps<T> taps(w.taps);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // records a wavefront takes at a time: 64, or its share of a short item
     constexpr uint32_t WAVES = BLK / 64;
@@ -530,7 +567,7 @@ __device__ __forceinline__ void add_item(const TArgs &t, const wp::WArgs &w, con
         } else if constexpr (K == 1) {
             if (lane < TAPS) {   // lanes without a tap sit out the whole loop
                 const uint32_t off = (uint32_t)(lane + (TILE - 1) * (lane / W));
-                const cpx<T> *lt = taps + lane;
+                const Taps<T> lt = taps.at((uint32_t)lane);
                 int r = 0;
                 for (; r + U <= n; r += U) {
                     cpx<T> tp[U];
@@ -558,7 +595,7 @@ __device__ __forceinline__ void add_item(const TArgs &t, const wp::WArgs &w, con
                     for (int j = 0; j < U; ++j) {
                         const uint32_t tb =
                             (uint32_t)__builtin_amdgcn_readlane((int)h.tap, min(r + j, n - 1));
-                        const cpx<T> *blk = taps + tb;
+                        const Taps<T> blk = taps.at(tb);
 #pragma unroll
                         for (int k = 0; k < KU; ++k)   // beyond the block: its last tap
                             tp[j][k] =
@@ -595,7 +632,7 @@ __device__ __forceinline__ void add_item(const TArgs &t, const wp::WArgs &w, con
         const int y = cell / ST, x = cell - y * ST;
         const double val = tile[comp * CELLS + cell];
         tile[comp * CELLS + cell] = 0.0;
-        if (val != 0.0) unsafeAtomicAdd(g + ((size_t)y * w.g.nx + x) * stride + comp, val);
+        if (val != 0.0) grid_add(g + ((size_t)y * w.g.nx + x) * stride + comp, val);
     }
 }
 
@@ -739,9 +776,10 @@ bool wtile_plan(wt::Plan &p, uint64_t samples, uint64_t spots, uint32_t half_lo,
     return true;
 }
 
-hipError_t wtile_grid(wt::TArgs t, const wt::Plan &p, void *ws, int mode, bool fp64,
-                      const uint8_t *widths, hipStream_t st, hipStream_t *side, int nside,
-                      hipEvent_t fork, hipEvent_t *join) {
+template <bool BATCH>
+static hipError_t grid_pass(wt::TArgs t, const wt::Plan &p, void *ws, int mode, bool fp64,
+                            const uint8_t *widths, hipStream_t st, hipStream_t *side, int nside,
+                            hipEvent_t fork, hipEvent_t *join) {
     unsigned char *b = static_cast<unsigned char *>(ws);
     t.nspots = (uint32_t)p.spots;
     t.half_lo = p.half_lo;
@@ -766,14 +804,14 @@ hipError_t wtile_grid(wt::TArgs t, const wt::Plan &p, void *ws, int mode, bool f
     const uint32_t blocks = (uint32_t)((samples + per - 1) / per);
     hipError_t e = fill_u32(t.count, p.slots, 0u, st);
     if (e == hipSuccess) e = fill_u32(t.item_count, 128, 0u, st);
-    if (e == hipSuccess) e = wt::prep<false>(t, mode, fp64, blocks, st, 0);
+    if (e == hipSuccess) e = wt::prep<BATCH>(t, mode, fp64, blocks, st, 0);
     if (e != hipSuccess) return e;
     size_t bytes = p.scan_bytes;
     e = hipcub::DeviceScan::ExclusiveSum(b + p.off_scan, bytes, t.count, t.start, (int)p.slots, st);
     if (e != hipSuccess) return e;
     wt::k_items<<<dim3((t.nspots + wt::BLOCK - 1) / wt::BLOCK, p.ncls), wt::BLOCK, 0, st>>>(t);
     e = hipGetLastError();
-    if (e == hipSuccess) e = wt::prep<false>(t, mode, fp64, blocks, st, 1);
+    if (e == hipSuccess) e = wt::prep<BATCH>(t, mode, fp64, blocks, st, 1);
     if (e != hipSuccess) return e;
     // one persistent launch per list, widest first, dealt over the streams
     if (nside) {
@@ -788,8 +826,8 @@ hipError_t wtile_grid(wt::TArgs t, const wt::Plan &p, void *ws, int mode, bool f
             any |= widths[h] != 0;
         if (!any) continue;
         const int on = turn++ % (nside + 1);
-        e = fp64 ? wt::launch_list<double, false>(t, (uint32_t)l, on ? side[on - 1] : st)
-                 : wt::launch_list<float, false>(t, (uint32_t)l, on ? side[on - 1] : st);
+        e = fp64 ? wt::launch_list<double, BATCH>(t, (uint32_t)l, on ? side[on - 1] : st)
+                 : wt::launch_list<float, BATCH>(t, (uint32_t)l, on ? side[on - 1] : st);
     }
     // joined also after a failed launch: later work on the stream must not overtake these
     for (int i = 0; i < nside; ++i) {
@@ -798,6 +836,14 @@ hipError_t wtile_grid(wt::TArgs t, const wt::Plan &p, void *ws, int mode, bool f
         if (e == hipSuccess) e = j;
     }
     return e;
+}
+
+hipError_t wtile_grid(const wt::TArgs &t, const wt::Plan &p, void *ws, int mode, bool fp64,
+                      const uint8_t *widths, hipStream_t st, hipStream_t *side, int nside,
+                      hipEvent_t fork, hipEvent_t *join) {
+    return t.w.facet_args
+               ? grid_pass<true>(t, p, ws, mode, fp64, widths, st, side, nside, fork, join)
+               : grid_pass<false>(t, p, ws, mode, fp64, widths, st, side, nside, fork, join);
 }
 
 }  // namespace bam
