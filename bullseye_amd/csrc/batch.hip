@@ -744,13 +744,13 @@ int build_plan(gridding_parameters *p, int mode, const bullseye_batch_facet *fac
     a.v_scale = -(double)((double)facets[0].ny * facets[0].cell_y * (double)ARCSEC_TO_RAD);
     HIP_TRY(pl.walk.ensure(walk_order_bytes()));
     a.time_inner = pl.walk.as<int>();
-    HIP_TRY(launch_walk_order(a, lv.walk_order, pl.walk.as<int>(), lv.stream));
     // sorted row table for the class kernels' sample preparation (rebuilt by every pass, see
     // enqueue_all; this copy serves the autotuner's single launches)
     pl.rows = (uint32_t)rows;
     HIP_TRY(pl.rowrec.ensure(std::max<size_t>(1, rows) * sizeof(RowRec)));
     a.rowrec = pl.rowrec.as<RowRec>();
     HIP_TRY(build_row_tables(a, pl.rows, false, pl.rowrec.as<RowRec>(), nullptr, lv.stream));
+    HIP_TRY(launch_walk_order(a, lv.walk_order, pl.walk.as<int>(), lv.stream));
 
     // per-facet accumulation grids, normalisation slots and geometry
     pl.fkind.resize(n);

@@ -8,15 +8,15 @@
 //    the contiguous run starting at f * 2W + W - m.  The lane that prepares a sample writes the
 //    two run offsets into its LDS record; a walking lane reads its u-tap and the W v-taps from
 //    the table, so the walk is loads + MACs;
-//  * 4-correlation modes split the correlations over lanes (CPL = 1 per lane on the FP32
-//    paths, 2 on the FP64 path), which cuts the accumulator registers per lane;
+//  * the correlations are split over lanes (CPL = 1 per lane on the FP32 paths, 2 on the FP64
+//    path), which cuts the accumulator registers per lane: 2 correlations at W = 7 (4 facets x
+//    1.8 M samples) took 752 us in one lane, 425 us in two;
 //  * FP32 compensated sums take one Kahan step per run of samples on an unchanged footprint:
-//    the run's products are chained by FMA onto -c and the result is added with the Kahan
-//    correction.  A run is at most one step of G samples long.  The leader lane of each quad
-//    (QUAD consecutive samples) decides once per step whether the quad's valid samples share
-//    one footprint, so the walking lanes read one flag per uniform quad; in a mixed quad each
-//    sample either extends the open run (same footprint) or closes it and opens one on its
-//    own footprint.  The error stays O(u) per term times the run length, independent of the
+//    the run's products are chained by FMA onto the negative of the Kahan correction (so one
+//    register is both) and the result is added with a new correction.  A run is at most RUN
+//    samples long.  The leader lane of each quad (QUAD consecutive samples) decides once per step
+//    whether the quad's valid samples share one footprint, so the walking lanes read one flag
+//    per uniform quad; in a mixed quad every sample is looked at.  The error stays O(u) per term times the run length, independent of the
 //    number of samples a register sums.
 // A lane group is W * NSPLIT lanes: lane (h, a) owns u-residue a and correlations
 // [h*CPL, (h+1)*CPL) of all W v-residues.  Each group's LDS records start on a different
@@ -61,9 +61,10 @@ __host__ __device__ constexpr uint32_t rot_table_len(uint32_t os, int w) {
 
 template <int MODE, int PATH, int W> struct GridderW {
     static constexpr int NC = ModeTraits<MODE>::NCORR;
-    // correlations per lane: one on the FP32 paths (fewest registers), two on the FP64 path
-    // (its double-width records make per-sample LDS reads the larger cost)
-    static constexpr int CPL = NC == 4 ? (PATH == PATH_FP64 ? 2 : 1) : NC;
+    // correlations per lane: one on the FP32 paths (fewest registers: two correlations of
+    // W = 7 in one lane took 205, two wavefronts a SIMD), two on the FP64 path (its double-width
+    // records make per-sample LDS reads the larger cost)
+    static constexpr int CPL = NC == 1 ? 1 : PATH == PATH_FP64 ? 2 : 1;
     static constexpr int NSPLIT = NC / CPL;
     static constexpr int G = W * NSPLIT;               // lanes per group
     static constexpr int GPW = 64 / G;                 // groups per wavefront
@@ -71,6 +72,13 @@ template <int MODE, int PATH, int W> struct GridderW {
     static constexpr bool KAHAN = PathTraits<PATH>::KAHAN;
     static constexpr bool TR = PATH != PATH_FP64;
     typedef Rec<T, NC, W, TR> R_t;
+    // Samples of a uniform quad that a compensated run chains (more than a quad: a whole step;
+    // otherwise a sample outside uniform quads is a run of its own).  The rounding of a run grows
+    // with its length, so the lengths keep the grids' distance from 64 bits: 2 correlations, W =
+    // 7: 3.3e-8 to 4.2e-8 of the rms (two draws of 1.8 M samples) with runs of a step, 2.7e-8 to
+    // 2.9e-8 with these (rounding the result alone: 2.5e-8).
+    static constexpr int RUN = NC == 4 ? G + QUAD : NC == 2 && W == 3 ? 1 : NC == 2 && W == 7 ? 2
+                                                                                             : QUAD;
     // bytes between the record arrays of consecutive groups: 16-byte aligned and starting
     // 8 banks (of 4 bytes, 32 banks) after the previous group
     static constexpr int GRAW = (G * (int)sizeof(R_t) + 15) & ~15;
@@ -259,10 +267,32 @@ template <int MODE, int PATH, int W> struct GridderW {
         return true;
     }
 
-    typedef acc1<T, KAHAN> Acc[W][CPL][2];
+    // A register sum.  Compensated: the true sum is s + n; a run's products are chained onto n,
+    // and one Kahan step ends the run.
+    struct Sum {
+        T s, n;
+        __device__ __forceinline__ void zero() { s = n = T(0); }
+        __device__ __forceinline__ void add(T x, T tap) {
+            if constexpr (KAHAN)
+                n = fma(x, tap, n);
+            else
+                s = fma(x, tap, s);
+        }
+        __device__ __forceinline__ void close() {
+            if constexpr (KAHAN) {
+                const T t = s + n;
+                n = n - (t - s);
+                s = t;
+            }
+        }
+        __device__ __forceinline__ double value() const {
+            return KAHAN ? (double)s + (double)n : (double)s;
+        }
+    };
+    typedef Sum Acc[W][CPL][2];
 
     // Adds one grid point's sums into the FP64 grid (skipped when they are zero) and clears them.
-    static __device__ __forceinline__ void flush1(double *cell, acc1<T, KAHAN> (&acc)[CPL][2]) {
+    static __device__ __forceinline__ void flush1(double *cell, Sum (&acc)[CPL][2]) {
         bool nz = false;
 #pragma unroll
         for (int k = 0; k < CPL; ++k) nz |= (acc[k][0].s != T(0)) | (acc[k][1].s != T(0));
@@ -295,7 +325,6 @@ template <int MODE, int PATH, int W> struct GridderW {
     static __device__ __forceinline__ void move_to(const GridArgs &a, uint32_t facet, int ua,
                                                    int c0, int x0, int y0, int cgi, int &px0,
                                                    int &py0, int &pcgi, Acc &acc) {
-        if (x0 == px0 && y0 == py0 && cgi == pcgi) return;
         if (pcgi >= 0) {
             const int xo = px0 + mod_w(ua - px0 % W);
             const bool all = (cgi != pcgi) || ((unsigned)(xo - x0) >= (unsigned)W);
@@ -328,7 +357,7 @@ template <int MODE, int PATH, int W> struct GridderW {
             return tap[rec.tu + ua];
     }
 
-    // One sample into the register sums (classic Kahan step on the compensated path).
+    // One sample on the sums' footprint.
     static __device__ __forceinline__ void add_one(const R_t &rec, const T *tap, int ua, int c0,
                                                    Acc &acc) {
         const T cu = u_tap(rec, tap, ua);
@@ -345,68 +374,21 @@ template <int MODE, int PATH, int W> struct GridderW {
             const T cv = cvp[r];
 #pragma unroll
             for (int k = 0; k < CPL; ++k) {
-                if constexpr (KAHAN) {
-                    acc[r][k][0].add_pre(vs[k].re * cv - acc[r][k][0].c);
-                    acc[r][k][1].add_pre(vs[k].im * cv - acc[r][k][1].c);
-                } else {
-                    acc[r][k][0].s = fma(vs[k].re, cv, acc[r][k][0].s);
-                    acc[r][k][1].s = fma(vs[k].im, cv, acc[r][k][1].s);
-                }
+                acc[r][k][0].add(vs[k].re, cv);
+                acc[r][k][1].add(vs[k].im, cv);
             }
         }
     }
 
-    typedef T Run[W][CPL][2];
-
-    // A run starts from -c of every register sum and ends with one Kahan step.
-    static __device__ __forceinline__ void open_run(const Acc &acc, Run &y) {
+    // Ends a run: one Kahan step of every register sum.
+    static __device__ __forceinline__ void close_run(Acc &acc) {
 #pragma unroll
         for (int r = 0; r < W; ++r)
 #pragma unroll
             for (int k = 0; k < CPL; ++k) {
-                y[r][k][0] = -acc[r][k][0].c;
-                y[r][k][1] = -acc[r][k][1].c;
+                acc[r][k][0].close();
+                acc[r][k][1].close();
             }
-    }
-
-    static __device__ __forceinline__ void close_run(Acc &acc, const Run &y) {
-#pragma unroll
-        for (int r = 0; r < W; ++r)
-#pragma unroll
-            for (int k = 0; k < CPL; ++k) {
-                acc[r][k][0].add_pre(y[r][k][0]);
-                acc[r][k][1].add_pre(y[r][k][1]);
-            }
-    }
-
-    // One sample on the run's footprint: its products chained by FMA onto the run.
-    static __device__ __forceinline__ void run_one(const R_t &rec, const T *tap, int ua, int c0,
-                                                   Run &y) {
-        const T cu = u_tap(rec, tap, ua);
-        const T *cvp = v_taps(rec, tap);
-        cpx<T> vs[CPL];
-#pragma unroll
-        for (int k = 0; k < CPL; ++k) {
-            vs[k] = rec.vis[c0 + k];
-            vs[k].re *= cu;
-            vs[k].im *= cu;
-        }
-#pragma unroll
-        for (int r = 0; r < W; ++r) {
-            const T cv = cvp[r];
-#pragma unroll
-            for (int k = 0; k < CPL; ++k) {
-                y[r][k][0] = fma(vs[k].re, cv, y[r][k][0]);
-                y[r][k][1] = fma(vs[k].im, cv, y[r][k][1]);
-            }
-        }
-    }
-
-    // QUAD samples on the run's footprint.
-    static __device__ __forceinline__ void run_quad(const R_t *recs, const T *tap, int ua, int c0,
-                                                    Run &y) {
-#pragma unroll
-        for (int q = 0; q < QUAD; ++q) run_one(recs[q], tap, ua, c0, y);
     }
 
     // Publication of the lanes' partial sums needs every lane of the wave: walk() may return
@@ -470,6 +452,16 @@ template <int MODE, int PATH, int W> struct GridderW {
             }
         int px0 = -1, py0 = -1, pcgi = -1;   // footprint of the accumulated samples
         int ncgi = -1;
+        // one sample; on another footprint than the last it ends the run and moves the ownership
+        auto add_moving = [&](const R_t &r) {
+            if (r.cgi < 0) return;
+            if (r.x0 != px0 || r.y0 != py0 || r.cgi != pcgi) {
+                if (RUN > QUAD) close_run(acc);
+                move_to(a, facet, ua, c0, r.x0, r.y0, r.cgi, px0, py0, pcgi, acc);
+            }
+            add_one(r, stap, ua, c0, acc);
+            if (RUN <= QUAD) close_run(acc);
+        };
 
         // this lane's sample s = step0 + gl as (outer, inner) indexes of the stream's
         // serpentine order (stream_sample), advanced by G samples a step without a division
@@ -574,49 +566,28 @@ template <int MODE, int PATH, int W> struct GridderW {
                     grp[gl].qcgi = cg;
                 }
                 if (!QUAD_LANES) wave_sync();
-                Run y;
-                bool open = false;
                 for (int q = 0; q < nq; ++q) {
                     const R_t &L = grp[q * QUAD];
                     if (L.qf) {
                         if (L.qcgi < 0) continue;   // no valid sample in the quad
-                        if (open && (L.qx0 != px0 || L.qy0 != py0 || L.qcgi != pcgi)) {
-                            close_run(acc, y);
-                            open = false;
-                        }
-                        if (!open) {
+                        if (L.qx0 != px0 || L.qy0 != py0 || L.qcgi != pcgi) {
+                            if (RUN > QUAD) close_run(acc);
                             move_to(a, facet, ua, c0, L.qx0, L.qy0, L.qcgi, px0, py0, pcgi, acc);
-                            open_run(acc, y);
-                            open = true;
                         }
-                        run_quad(grp + q * QUAD, stap, ua, c0, y);
-                    } else {
-                        // a mixed quad: a sample on the open run's footprint extends the run;
-                        // one elsewhere closes it, moves the ownership and opens a new run
 #pragma unroll
                         for (int k2 = 0; k2 < QUAD; ++k2) {
-                            const R_t &rr = grp[q * QUAD + k2];
-                            if (rr.cgi < 0) continue;
-                            if (!open || rr.x0 != px0 || rr.y0 != py0 || rr.cgi != pcgi) {
-                                if (open) close_run(acc, y);
-                                move_to(a, facet, ua, c0, rr.x0, rr.y0, rr.cgi, px0, py0, pcgi,
-                                        acc);
-                                open_run(acc, y);
-                                open = true;
-                            }
-                            run_one(rr, stap, ua, c0, y);
+                            add_one(grp[q * QUAD + k2], stap, ua, c0, acc);
+                            if (RUN <= QUAD && k2 % RUN == RUN - 1) close_run(acc);
                         }
+                    } else {
+#pragma unroll
+                        for (int k2 = 0; k2 < QUAD; ++k2) add_moving(grp[q * QUAD + k2]);
                     }
                 }
-                if (open) close_run(acc, y);
                 kk = nq * QUAD;
             }
-            for (; kk < kmax; ++kk) {
-                const int cg = grp[kk].cgi;
-                if (cg < 0) continue;
-                move_to(a, facet, ua, c0, grp[kk].x0, grp[kk].y0, cg, px0, py0, pcgi, acc);
-                add_one(grp[kk], stap, ua, c0, acc);
-            }
+            for (; kk < kmax; ++kk) add_moving(grp[kk]);
+            if (RUN > QUAD) close_run(acc);
             wave_sync();
             si += dsi;
             so += dso;
@@ -907,8 +878,14 @@ constexpr bool one_per_wave(int mode, int path, int W) {
     return W == 7 && path != PATH_FP64 && (mode == MODE_4 || mode == MODE_4J);
 }
 
+// Wavefronts a SIMD should hold, where the registers stay without spills for it.
+constexpr int min_waves(int mode, int path, int W) {
+    const bool four = mode == MODE_4 || mode == MODE_4J;
+    return one_per_wave(mode, path, W) || (!four && path != PATH_FP64 && W <= 9) ? 4 : 1;
+}
+
 template <int MODE, int PATH, int W>
-__global__ __launch_bounds__(BLOCK, one_per_wave(MODE, PATH, W) ? 4 : 1)
+__global__ __launch_bounds__(BLOCK, min_waves(MODE, PATH, W))
 void romein_w_kernel(GridArgs a) {
     typedef GridderW<MODE, PATH, W> Gd;
     typedef typename Gd::T T;
@@ -985,7 +962,7 @@ hipError_t launch_romein_aa(const GridArgs &a, int mode, int path, hipStream_t s
 // Lane groups per wavefront for a support width, or 0 when no specialisation exists.
 int romein_w_groups_per_wave(int W, int mode, int path) {
     if (rw::one_per_wave(mode, path, W)) return 1;
-    const int split = (mode == MODE_4 || mode == MODE_4J) ? (path == PATH_FP64 ? 2 : 4) : 1;
+    const int split = (mode == MODE_4 || mode == MODE_4J) ? (path == PATH_FP64 ? 2 : 4) : mode == MODE_2 && path != PATH_FP64 ? 2 : 1;
     switch (W) {
         case 3: case 5: case 7: case 9: case 11: return 64 / (W * split);
     }

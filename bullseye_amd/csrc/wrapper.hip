@@ -307,16 +307,22 @@ static void choose_streams(const gridding_parameters *p, size_t F, size_t B, siz
         const size_t per_bl = std::max<size_t>(1, rows / std::max<size_t>(1, B));
         nseg = (uint32_t)std::max<size_t>(1, per_bl / g.opts.rows_per_stream);
     } else {
-        // enough lane groups to fill 256 CUs x 4 SIMDs several waves deep, segments of at least
-        // 8 rows (one facet of 2016 baselines x 240 rows x 16 channels: 15-row segments grid in
-        // 0.44 ms, 30-row ones in 0.59 ms, 8-row ones in 0.51 ms)
+        // enough lane groups for the wavefronts that 256 CUs x 4 SIMDs hold together (4 a SIMD,
+        // 2 of the FP64 path's 4-correlation kernels: 7 facets of 351 baselines x 101 rows at
+        // W = 9 take 1.10 ms with rows for 4, 1.04 ms with rows for 2), in segments of at least 8
+        // rows (one facet of 2016 baselines x 240 rows x 16 channels: 15-row segments grid in
+        // 0.40 ms, 30-row ones in 0.54 ms, 8-row ones in 0.51 ms) and 32 samples, since every
+        // segment gives up a whole footprint (a cube of one channel a slice, 351 baselines x 150
+        // rows: 364 us a call with 19 samples a segment, 326 us with 38)
         int gpw = romein_w_groups_per_wave(W, mode, g.path);
         if (gpw == 0) gpw = 64 / std::max(1, W * ((W + 7) / 8));
-        const size_t want_groups = (size_t)256 * 4 * 4 * gpw;
+        const bool wide = g.path == PATH_FP64 && (mode == MODE_4 || mode == MODE_4J);
+        const size_t want_groups = (size_t)256 * 4 * (wide ? 2 : 4) * gpw;
         const size_t have = F * B * nblocks;
+        const size_t least = std::max<size_t>(8, (32 + cps - 1) / cps);
         nseg = 1;
         const size_t per_bl = std::max<size_t>(1, rows / std::max<size_t>(1, B));
-        while (have * nseg < want_groups && per_bl / (nseg * 2) >= 8) nseg *= 2;
+        while (have * nseg < want_groups && per_bl / (nseg * 2) >= least) nseg *= 2;
     }
 }
 
@@ -706,7 +712,6 @@ static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
     void *walk;
     HIP_TRY(table(g.walk, walk_order_bytes(), &walk));
     a.time_inner = (const int *)walk;
-    HIP_TRY(launch_walk_order(a, (int)g.opts.walk_order, (int *)walk, g.stream));
 
     // sorted row table (every gridder's sample preparation) and channel table (the AA gridder)
     {
@@ -720,6 +725,7 @@ static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
         HIP_TRY(build_row_tables(a, (uint32_t)rows, mode == MODE_4J && rows > 0,
                                  (RowRec *)rowrec, (ChanRec *)chanrec, g.stream));
     }
+    HIP_TRY(launch_walk_order(a, (int)g.opts.walk_order, (int *)walk, g.stream));
 
     if (wproj) {
         const float wmax_f = (float)p->wmax_est;
