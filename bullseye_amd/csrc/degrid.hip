@@ -303,6 +303,11 @@ template <typename T> __device__ __forceinline__ T xor_lane(T v, int mask) {
 }
 
 // Any kernel: the wavefront sums the footprints of its 64 samples one after the other.
+// What bounds it is the latency of taps and grid cells, so the first 64 taps of GROUP samples are
+// loaded together, then the rest of the wide ones AHEAD loads at a time.  One million w-projected
+// samples: 489 us with sixteen lanes a sample and 639 with one sample's loads at a time on a
+// spread observation (1.3e8 taps), 359 with this; on 4 timesteps of 8128 baselines 263, 151 and
+// 162 us.
 template <int MODE, int PATH, bool WPROJ>
 __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     constexpr int NC = ModeTraits<MODE>::NCORR;
@@ -319,47 +324,96 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     cpx<T> acc[NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k) acc[k] = {T(0), T(0)};
+    constexpr int WORDS = NC * (int)sizeof(T) / 4;
+    constexpr int GROUP = WORDS <= 1 ? 8 : WORDS <= 2 ? 4 : 2, AHEAD = WORDS <= 2 ? 4 : 2;
+    // The footprint of the sample of lane r, in scalar registers (one tap of the table and the
+    // grid's first cell where the sample does not count).
+    struct Footprint {
+        uint32_t wp, tb, ntap, inv, cg;
+        int x0, y0, fu, fv;
+        __device__ __forceinline__ Footprint(const Place<T> &p, uint32_t cgi,
+                                             uint32_t lane_inv, int r, uint64_t on) {
+            const bool live = (on >> r) & 1;
+            wp = live ? (uint32_t)__builtin_amdgcn_readlane(p.wp, r) : 1u;
+            tb = live ? (uint32_t)__builtin_amdgcn_readlane((int)p.tb, r) : 0u;
+            x0 = live ? __builtin_amdgcn_readlane(p.x0, r) : 0;
+            y0 = live ? __builtin_amdgcn_readlane(p.y0, r) : 0;
+            fu = live ? __builtin_amdgcn_readlane(p.fu, r) : 0;
+            fv = live ? __builtin_amdgcn_readlane(p.fv, r) : 0;
+            cg = live ? (uint32_t)__builtin_amdgcn_readlane((int)cgi, r) : 0u;
+            inv = live ? (uint32_t)__builtin_amdgcn_readlane((int)lane_inv, r) : 0u;
+            ntap = wp * wp;
+        }
+    };
+    // Tap t of a footprint (conjugated) and the grid values under it.
+    auto load_tap = [&](const Footprint &q, uint32_t f, uint32_t t, cpx<T> &tap, cpx<T> (&gv)[NC]) {
+        const uint32_t y = (t * q.inv) >> 20, x = t - y * q.wp;
+        if constexpr (WPROJ) {
+            const cpx<T> tw = wtaps[q.tb + t];
+            tap = {tw.re, -tw.im};
+        } else {
+            tap = {conv[q.fu + x * a.OS] * conv[q.fv + y * a.OS], T(0)};
+        }
+        const grid_base_type *cell = slice_of(d, f, q.cg) +
+                                     2 * ((size_t)q.y0 * a.nx + (size_t)q.x0) +
+                                     2 * ((size_t)y * a.nx + x);
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+            gv[k] = {(T)cell[2 * (size_t)k * slice], (T)cell[2 * (size_t)k * slice + 1]};
+    };
     for (uint32_t f = 0; f < a.facets; ++f) {
         const Place<T> p = place<MODE, PATH, WPROJ>(d, sm, f);
         const uint64_t on = __ballot(p.on);
+        const uint64_t wide = __ballot(p.on && p.wp * p.wp > 64);
+        // t / wp for t < 64^2: t * (2^20 / wp + 1) >> 20 is exact (t times the reciprocal's excess
+        // stays below 2^20)
+        const uint32_t inv = p.on ? (1u << 20) / (uint32_t)p.wp + 1 : 0u;
         for (int r0 = 0; r0 < 64; r0 += PACK) {
             if (!((on >> r0) & ((1ull << PACK) - 1))) continue;
             cpx<T> part[PACK][NC];
+            // a sample's first 64 taps: the loads of GROUP samples leave together
 #pragma unroll
-            for (int j = 0; j < PACK; ++j) {
+            for (int j0 = 0; j0 < PACK; j0 += GROUP) {
+                cpx<T> tap[GROUP], gv[GROUP][NC];
+                bool mine_too[GROUP];
 #pragma unroll
-                for (int k = 0; k < NC; ++k) part[j][k] = {T(0), T(0)};
-                const int r = r0 + j;
-                if (!((on >> r) & 1)) continue;
-                // the sample's place, in scalar registers
-                const uint32_t wp = (uint32_t)__builtin_amdgcn_readlane(p.wp, r);
-                const uint32_t tb = (uint32_t)__builtin_amdgcn_readlane((int)p.tb, r);
-                const int x0 = __builtin_amdgcn_readlane(p.x0, r);
-                const int y0 = __builtin_amdgcn_readlane(p.y0, r);
-                const int fu = __builtin_amdgcn_readlane(p.fu, r);
-                const int fv = __builtin_amdgcn_readlane(p.fv, r);
-                const uint32_t cg = (uint32_t)__builtin_amdgcn_readlane((int)sm.cgi, r);
-                const grid_base_type *g = slice_of(d, f, cg) + 2 * ((size_t)y0 * a.nx + (size_t)x0);
-                // t / wp for t < 64^2: t * (2^20 / wp + 1) >> 20 is exact (t times the
-                // reciprocal's excess stays below 2^20)
-                const uint32_t inv = (1u << 20) / wp + 1;
-                const uint32_t ntap = wp * wp;
-                for (uint32_t t = (uint32_t)lane; t < ntap; t += 64) {
-                    const uint32_t y = (t * inv) >> 20, x = t - y * wp;
-                    cpx<T> tap;   // conjugated
-                    if constexpr (WPROJ) {
-                        const cpx<T> tw = wtaps[tb + t];
-                        tap = {tw.re, -tw.im};
-                    } else {
-                        tap = {conv[fu + x * a.OS] * conv[fv + y * a.OS], T(0)};
-                    }
-                    const grid_base_type *cell = g + 2 * ((size_t)y * a.nx + x);
+                for (int j = 0; j < GROUP; ++j) {
+                    const Footprint q(p, sm.cgi, inv, r0 + j0 + j, on);
+                    mine_too[j] = (uint32_t)lane < q.ntap;
+                    load_tap(q, f, min((uint32_t)lane, q.ntap - 1), tap[j], gv[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < GROUP; ++j)
 #pragma unroll
                     for (int k = 0; k < NC; ++k) {
-                        const cpx<T> gv = {(T)cell[2 * (size_t)k * slice],
-                                           (T)cell[2 * (size_t)k * slice + 1]};
-                        part[j][k] = cmac(part[j][k], tap, gv);
+                        const cpx<T> v = cmac(cpx<T>{T(0), T(0)}, tap[j], gv[j][k]);
+                        part[j0 + j][k].re = mine_too[j] ? v.re : T(0);
+                        part[j0 + j][k].im = mine_too[j] ? v.im : T(0);
                     }
+            }
+            // the taps beyond, AHEAD loads in flight while there are that many
+#pragma unroll
+            for (int j = 0; j < PACK; ++j) {
+                if (!((wide >> (r0 + j)) & 1)) continue;
+                const Footprint q(p, sm.cgi, inv, r0 + j, on);
+                uint32_t t0 = 64;
+                for (; t0 + 64 < q.ntap; t0 += 64 * AHEAD) {
+                    cpx<T> tap[AHEAD], gv[AHEAD][NC];
+#pragma unroll
+                    for (int h = 0; h < AHEAD; ++h)
+                        load_tap(q, f, min(t0 + 64 * h + (uint32_t)lane, q.ntap - 1), tap[h], gv[h]);
+#pragma unroll
+                    for (int h = 0; h < AHEAD; ++h)
+                        if (t0 + 64 * h + (uint32_t)lane < q.ntap)
+#pragma unroll
+                            for (int k = 0; k < NC; ++k)
+                                part[j][k] = cmac(part[j][k], tap[h], gv[h][k]);
+                }
+                if (t0 < q.ntap && t0 + (uint32_t)lane < q.ntap) {
+                    cpx<T> tap, gv[NC];
+                    load_tap(q, f, t0 + (uint32_t)lane, tap, gv);
+#pragma unroll
+                    for (int k = 0; k < NC; ++k) part[j][k] = cmac(part[j][k], tap, gv[k]);
                 }
             }
             // reduce: at each of three steps a lane keeps the half of the samples that its bit

@@ -91,8 +91,8 @@ hipError_t ingest_sort(const uint32_t *a1, const uint32_t *a2, uint32_t rows, ui
 // so the result is the same on every run.  The flag stays on the device for the gridding
 // kernels.  override_order: 1 channels inner, 2 time inner, anything else measured.
 // A thread a baseline, 33 rows in turn, took 33 us from 351 baselines to 2016; this takes 7 us.
-constexpr int WALK_BLOCKS = 256;
-constexpr int WALK_THREADS = 256;
+constexpr int WALK_BLOCKS = 64;
+constexpr int WALK_THREADS = 1024;
 constexpr uint32_t WALK_ROWS = 33;
 
 // 1 / wavelength of the middle channel pair of a row, and its u, v in cells times wavelength.

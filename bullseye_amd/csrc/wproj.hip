@@ -7,6 +7,10 @@
 // 2S+3 of the high grid edge is dropped; tap (j, k) of the footprint is
 // conv[plane][frac_v + j*OS][frac_u + k*OS]; the normalisation adds weight * sum Re(taps).
 //
+// Where these kernels run: most calls and batches go through on-chip tiles (wtile.hip); these class
+// kernels grid the calls whose samples or bins one tiled pass cannot number, the batches whose
+// autotuned tiles are faster, a batch's per-facet schedule, and the calls that ask for them.
+//
 // Variable support.  Each plane p carries its own half support S_p <= S (S = conv_support):
 // its taps outside [S - S_p, S + S_p] are taken as zero (the kernel generator truncates them), so
 // only the W_p x W_p centre of the (2S+1)^2 footprint is walked.  At initLibrary the taps are

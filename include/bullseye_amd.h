@@ -348,8 +348,8 @@ typedef struct bullseye_batch_facet {
 } bullseye_batch_facet;
 
 enum bullseye_batch_schedule {
-    BULLSEYE_BATCH_PERSISTENT_GRAPH = 0, /* one persistent launch per (kind, support class) over
-                                            all facets, captured in a HIP graph and replayed */
+    BULLSEYE_BATCH_PERSISTENT_GRAPH = 0, /* persistent launches over all facets, captured in a
+                                            HIP graph and replayed */
     BULLSEYE_BATCH_PERSISTENT = 1,       /* the same launches issued on the stream each time */
     BULLSEYE_BATCH_PER_FACET = 2         /* one launch per (facet, support class), issued on the
                                             stream each time: the unbatched baseline */
@@ -359,7 +359,8 @@ enum bullseye_batch_schedule {
  * (0 default, 1 column ownership (M <= 15), 2/3/4 residue pairs with at least 1/2/4 pairs per
  * lane) and chunk[i] the classification segments per work item (1, 2 or 4: the visibility
  * chunk length is chunk * base_rows rows).  channels_per_stream and base_rows are shared by all
- * classes (0: automatic, 32). */
+ * classes (0: automatic, 32).  With every shape at 0, every chunk at most 1 and facet_major 0 the
+ * facets run through on-chip tiles instead of the class kernels these choices are for. */
 typedef struct bullseye_batch_tuning {
     uint32_t struct_size;       /* sizeof(bullseye_batch_tuning) */
     uint32_t channels_per_stream;
