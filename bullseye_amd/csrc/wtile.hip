@@ -10,6 +10,8 @@
 // memory side whatever they carry.  Here a tile of 4096 samples of 49 taps costs about 400
 // requests (0.002 per tap), the adds are LDS atomics (ds_add_f64: 8.7 cycles per wavefront on
 // consecutive doubles, 4.5 T adds/s over the chip), and no lane owns or moves anything.
+// Measured: 125 M samples on 4096^2 (supports 7..63) 41 -> 11.2 ms a call, of which the LDS adds
+// take 6.2 ms and the two preparing passes 2.9 ms; 0.4 M samples into two facets 1.64 -> 0.50 ms.
 //
 //   k_count    bin of every sample, counted (one atomic per bin and wavefront)
 //   scan       first record of every bin
