@@ -11,18 +11,23 @@
 //   S = Pinv^H S Qinv in the Jones mode (the forward applies V -> Pinv V Qinv^H),
 // and out[row][chan][corr_k] = sum over facets of s_k; every other correlation is zero.
 //
-// A gather: no atomics.  One lane prepares one (row, channel) sample per facet (the FP64 geometry
-// and rotor, 200 instructions, once: a group of 16 lanes sharing a sample repeated them 16
-// times and was bound by that).  The taps are then summed
-//   AA, W = 3..11   by the sample's own lane: both tap runs in registers, the model read in
-//                   rows of W complex values; neighbouring lanes are neighbouring channels, whose
-//                   footprints share cache lines.  9 instructions a sample's tap row and
-//                   correlation, and no exchange between lanes (6 facets x 4 correlations,
-//                   1.01 M samples: 1.69 -> 0.38 ms a call).
-//   others          by the wavefront, sample after sample: a sample's w-kernel block is W_p x W_p
-//                   consecutive taps, which lanes of their own samples could only read line by
-//                   line.  Eight samples' partial sums are reduced together (each exchange halves
-//                   the samples a lane keeps: 10 exchanges for eight, not 6 for each).
+// A gather: no atomics.  Three ways to sum a sample's taps; launch_t says which and why.
+//   degrid_aa_kernel     AA, W = 3..11: a lane a sample.  The FP64 geometry and rotor (200
+//                        instructions) are prepared once, both tap runs sit in registers, the
+//                        model is read in rows of W complex values; neighbouring lanes are
+//                        neighbouring channels, whose footprints share cache lines.  9
+//                        instructions a sample's tap row and correlation, no exchange between
+//                        lanes (6 facets x 4 correlations, 1.01 M samples: 1.69 -> 0.38 ms a call
+//                        against sixteen lanes a sample).
+//   degrid_wave_kernel   w-projection, large calls: a wavefront sums the footprints of its 64
+//                        samples one after the other, since a sample's w-kernel block is W_p x
+//                        W_p consecutive taps, which lanes of their own samples could only read
+//                        line by line.  Eight samples' partial sums are reduced together (each
+//                        exchange halves the samples a lane keeps: 10 exchanges for eight, not 6
+//                        for each).
+//   degrid_group_kernel  everything else: sixteen lanes a sample, every one of which prepares it.
+//                        The preparation is repeated, but a call has sixteen times as many
+//                        wavefronts in flight and a sample's chain of loads is short.
 #include "device_common.h"
 
 namespace bam {
@@ -30,6 +35,7 @@ namespace dg {
 
 constexpr int BLOCK = 256;
 constexpr int PACK = 8;     // samples reduced together
+constexpr int GL = 16;      // lanes a sample of degrid_group_kernel
 
 struct DArgs {
     GridArgs g;                      // inputs and geometry (g.grid and g.norm unused)
@@ -42,6 +48,7 @@ struct DArgs {
     float wmax_f;
     uint32_t P;                      // correlation slices per (facet, cube) group
     uint64_t rows;
+    uint64_t first;                  // first sample of the launch
 };
 
 // One sample: what does not depend on the facet.
@@ -260,7 +267,7 @@ __global__ __launch_bounds__(BLOCK) void degrid_aa_kernel(DArgs d) {
         conv[i] = reinterpret_cast<const T *>(a.conv)[i];
     __syncthreads();
     Sample<MODE, PATH> sm;
-    sm.load(d, (uint64_t)blockIdx.x * BLOCK + threadIdx.x);
+    sm.load(d, d.first + (uint64_t)blockIdx.x * BLOCK + threadIdx.x);
     const size_t slice = (size_t)a.nx * a.ny;
     cpx<T> acc[NC];
 #pragma unroll
@@ -298,17 +305,83 @@ __global__ __launch_bounds__(BLOCK) void degrid_aa_kernel(DArgs d) {
     store(d, sm, acc);
 }
 
+template <typename T> __device__ __forceinline__ T group_sum(T v) {
+#pragma unroll
+    for (int o = GL / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, GL);
+    return v;
+}
+
+// Wavefronts a SIMD the group kernel is scheduled for.  FP64 with Jones terms: scheduled for four
+// (124 registers) its loads wait for each other, 2.06 M samples of a W <= 15 stack take 4.8 ms
+// against 4.2 with three (142 registers).
+constexpr int group_waves(int mode, int path) {
+    return mode == MODE_4J && path == PATH_FP64 ? 3 : 8;
+}
+
+// Any kernel: GL lanes a sample, their partial sums added by a butterfly.
+template <int MODE, int PATH, bool WPROJ>
+__global__ __launch_bounds__(BLOCK)
+__attribute__((amdgpu_waves_per_eu(1, group_waves(MODE, PATH)))) void degrid_group_kernel(DArgs d) {
+    constexpr int NC = ModeTraits<MODE>::NCORR;
+    typedef typename PathTraits<PATH>::acc_t T;
+    const GridArgs &a = d.g;
+    const int gl = (int)(threadIdx.x % GL);
+    Sample<MODE, PATH> sm;
+    sm.load(d, d.first + ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) / GL);
+    const size_t slice = (size_t)a.nx * a.ny;
+    const T *conv = reinterpret_cast<const T *>(a.conv);
+    const cpx<T> *wtaps = reinterpret_cast<const cpx<T> *>(d.taps);
+    cpx<T> acc[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[k] = {T(0), T(0)};
+    for (uint32_t f = 0; f < a.facets; ++f) {
+        const Place<T> p = place<MODE, PATH, WPROJ>(d, sm, f);
+        cpx<T> sk[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) sk[k] = {T(0), T(0)};
+        if (p.on) {
+            const grid_base_type *g =
+                slice_of(d, f, sm.cgi) + 2 * ((size_t)p.y0 * a.nx + (size_t)p.x0);
+            const int ntap = p.wp * p.wp;
+            for (int t = gl; t < ntap; t += GL) {
+                const int y = t / p.wp, x = t - y * p.wp;
+                cpx<T> tap;
+                if constexpr (WPROJ) {
+                    tap = conjg(wtaps[p.tb + (uint32_t)t]);
+                } else {
+                    tap = {conv[p.fu + x * (int)a.OS] * conv[p.fv + y * (int)a.OS], T(0)};
+                }
+                const grid_base_type *cell = g + 2 * ((size_t)y * a.nx + (size_t)x);
+#pragma unroll
+                for (int k = 0; k < NC; ++k) {
+                    const cpx<T> gv = {(T)cell[2 * (size_t)k * slice],
+                                       (T)cell[2 * (size_t)k * slice + 1]};
+                    sk[k] = cadd(sk[k], cmul(tap, gv));
+                }
+            }
+        }
+        // the whole group takes part, samples that are off included
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            sk[k].re = group_sum(sk[k].re);
+            sk[k].im = group_sum(sk[k].im);
+        }
+        if (p.on) finish(d, sm, p, f, sk, acc);
+    }
+    if (gl == 0) store(d, sm, acc);
+}
+
 template <typename T> __device__ __forceinline__ T xor_lane(T v, int mask) {
     return __shfl_xor(v, mask, 64);
 }
 
-// Any kernel: the wavefront sums the footprints of its 64 samples one after the other.
+// W-projection: the wavefront sums the footprints of its 64 samples one after the other.
 // What bounds it is the latency of taps and grid cells, so the first 64 taps of GROUP samples are
 // loaded together, then the rest of the wide ones AHEAD loads at a time.  One million w-projected
-// samples: 489 us with sixteen lanes a sample and 639 with one sample's loads at a time on a
-// spread observation (1.3e8 taps), 359 with this; on 4 timesteps of 8128 baselines 263, 151 and
-// 162 us.
-template <int MODE, int PATH, bool WPROJ>
+// samples, one correlation: 489 us with sixteen lanes a sample and 639 with one sample's loads at
+// a time on a spread observation (1.3e8 taps), 359 with this; on 4 timesteps of 8128 baselines
+// 263, 151 and 162 us.
+template <int MODE, int PATH>
 __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     constexpr int NC = ModeTraits<MODE>::NCORR;
     typedef typename PathTraits<PATH>::acc_t T;
@@ -317,9 +390,8 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     const int lane = threadIdx.x & 63;
     cpx<T>(*mine)[NC] = res[threadIdx.x >> 6];
     Sample<MODE, PATH> sm;
-    sm.load(d, (uint64_t)blockIdx.x * BLOCK + threadIdx.x);
+    sm.load(d, d.first + (uint64_t)blockIdx.x * BLOCK + threadIdx.x);
     const size_t slice = (size_t)a.nx * a.ny;
-    const T *conv = reinterpret_cast<const T *>(a.conv);
     const cpx<T> *wtaps = reinterpret_cast<const cpx<T> *>(d.taps);
     cpx<T> acc[NC];
 #pragma unroll
@@ -330,7 +402,7 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     // grid's first cell where the sample does not count).
     struct Footprint {
         uint32_t wp, tb, ntap, inv, cg;
-        int x0, y0, fu, fv;
+        int x0, y0;
         __device__ __forceinline__ Footprint(const Place<T> &p, uint32_t cgi,
                                              uint32_t lane_inv, int r, uint64_t on) {
             const bool live = (on >> r) & 1;
@@ -338,8 +410,6 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
             tb = live ? (uint32_t)__builtin_amdgcn_readlane((int)p.tb, r) : 0u;
             x0 = live ? __builtin_amdgcn_readlane(p.x0, r) : 0;
             y0 = live ? __builtin_amdgcn_readlane(p.y0, r) : 0;
-            fu = live ? __builtin_amdgcn_readlane(p.fu, r) : 0;
-            fv = live ? __builtin_amdgcn_readlane(p.fv, r) : 0;
             cg = live ? (uint32_t)__builtin_amdgcn_readlane((int)cgi, r) : 0u;
             inv = live ? (uint32_t)__builtin_amdgcn_readlane((int)lane_inv, r) : 0u;
             ntap = wp * wp;
@@ -348,12 +418,7 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     // Tap t of a footprint (conjugated) and the grid values under it.
     auto load_tap = [&](const Footprint &q, uint32_t f, uint32_t t, cpx<T> &tap, cpx<T> (&gv)[NC]) {
         const uint32_t y = (t * q.inv) >> 20, x = t - y * q.wp;
-        if constexpr (WPROJ) {
-            const cpx<T> tw = wtaps[q.tb + t];
-            tap = {tw.re, -tw.im};
-        } else {
-            tap = {conv[q.fu + x * a.OS] * conv[q.fv + y * a.OS], T(0)};
-        }
+        tap = conjg(wtaps[q.tb + t]);
         const grid_base_type *cell = slice_of(d, f, q.cg) +
                                      2 * ((size_t)q.y0 * a.nx + (size_t)q.x0) +
                                      2 * ((size_t)y * a.nx + x);
@@ -362,11 +427,11 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
             gv[k] = {(T)cell[2 * (size_t)k * slice], (T)cell[2 * (size_t)k * slice + 1]};
     };
     for (uint32_t f = 0; f < a.facets; ++f) {
-        const Place<T> p = place<MODE, PATH, WPROJ>(d, sm, f);
+        const Place<T> p = place<MODE, PATH, true>(d, sm, f);
         const uint64_t on = __ballot(p.on);
         const uint64_t wide = __ballot(p.on && p.wp * p.wp > 64);
-        // t / wp for t < 64^2: t * (2^20 / wp + 1) >> 20 is exact (t times the reciprocal's excess
-        // stays below 2^20)
+        // t / wp as t * (2^20 / wp + 1) >> 20: exact while t times the reciprocal's excess (at most
+        // 1) stays below 2^20 / wp, and t < wp^2 <= 63^2 with 63^3 < 2^20
         const uint32_t inv = p.on ? (1u << 20) / (uint32_t)p.wp + 1 : 0u;
         for (int r0 = 0; r0 < 64; r0 += PACK) {
             if (!((on >> r0) & ((1ull << PACK) - 1))) continue;
@@ -454,26 +519,60 @@ __global__ __launch_bounds__(BLOCK) void degrid_wave_kernel(DArgs d) {
     store(d, sm, acc);
 }
 
-template <int MODE, int PATH> static hipError_t launch_t(const DArgs &d, hipStream_t st) {
-    const uint64_t blocks = (d.rows * d.g.chan + BLOCK - 1) / BLOCK;
-    if (!blocks) return hipSuccess;
-    if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    const dim3 g((uint32_t)blocks), b(BLOCK);
+// Which kernel sums the taps.  Measured against sixteen lanes a sample (us a call, 512^2 grids,
+// w-kernels of up to 7, 15, 31 and 63 taps a side, samples in thousands):
+//   one correlation, FP32:  238: 47/37, 56/66, 99/108, 285/325   499: 101/63, 124/107, 192/168,
+//                           431/390; FP64 the wavefronts lead from 238 on (499: 159/86 .. 672/501)
+//   two correlations:       126: 32/33 and 238: 57/46 up to 7 a side; above, 499: 146/140, 218/234,
+//                           490/621   2064: 559/466, 814/730, 1807/1649
+//   four, FP32:             238: 88/84 up to 7; above, 980: 388/373, 571/600, 1239/1550   4128:
+//                           1531/1400, 2252/2142, 5324/5273; FP64 never (4128: 2468/2656 ..
+//                           14894/15147)
+// so wavefronts take the calls that are large enough to fill the GPU with them.  A lane a sample
+// (AA) lags only where its few wavefronts leave each with a long chain: 7 thousand samples of four
+// correlations 10/12 (W = 7) and 11/18 (W = 11), 15 thousand 12/12 and 15/18, 30 thousand 17/12 and
+// 24/19; two correlations 10/12, 13/12 and 18/13 at W = 11.
+template <int MODE, int PATH> static uint64_t wave_samples(uint32_t S) {
+    constexpr int NC = ModeTraits<MODE>::NCORR;
+    if (NC == 4 && PATH == PATH_FP64) return ~0ull;
+    if (S <= 3) return 1u << 17;   // a footprint in one load
+    return NC == 1 ? (PATH == PATH_FP64 ? 1u << 18 : 3u << 17) : NC == 2 ? 1u << 20 : 1u << 21;
+}
+
+template <int MODE, int PATH> static hipError_t launch_t(DArgs d, hipStream_t st) {
+    constexpr int NC = ModeTraits<MODE>::NCORR;
+    const uint64_t samples = d.rows * d.g.chan;
     const size_t smem = (size_t)d.g.csz * sizeof(typename PathTraits<PATH>::acc_t);
-    if (d.wproj)
-        degrid_wave_kernel<MODE, PATH, true><<<g, b, 0, st>>>(d);
-    else if (smem > 32768)   // an oversampling far beyond use: the taps stay in memory
-        degrid_wave_kernel<MODE, PATH, false><<<g, b, 0, st>>>(d);
-    else
-        switch (d.g.W) {
-            case 3: degrid_aa_kernel<MODE, PATH, 3><<<g, b, smem, st>>>(d); break;
-            case 5: degrid_aa_kernel<MODE, PATH, 5><<<g, b, smem, st>>>(d); break;
-            case 7: degrid_aa_kernel<MODE, PATH, 7><<<g, b, smem, st>>>(d); break;
-            case 9: degrid_aa_kernel<MODE, PATH, 9><<<g, b, smem, st>>>(d); break;
-            case 11: degrid_aa_kernel<MODE, PATH, 11><<<g, b, smem, st>>>(d); break;
-            default: degrid_wave_kernel<MODE, PATH, false><<<g, b, 0, st>>>(d);
+    const bool wave = d.wproj && samples >= wave_samples<MODE, PATH>(d.g.S);
+    const bool lane = !d.wproj && smem <= 32768 && (d.g.W & 1) && d.g.W >= 3 && d.g.W <= 11 &&
+                      (NC == 1 || samples >= 5120u * NC);
+    // a launch holds fewer than 2^32 work items
+    const uint64_t piece = wave || lane ? 1ull << 31 : 1ull << 27;
+    const dim3 b(BLOCK);
+    for (d.first = 0; d.first < samples; d.first += piece) {
+        const uint64_t n = samples - d.first < piece ? samples - d.first : piece;
+        const uint64_t lanes = wave || lane ? n : n * GL;
+        const dim3 g((uint32_t)((lanes + BLOCK - 1) / BLOCK));
+        if (wave) {
+            if constexpr (NC != 4 || PATH != PATH_FP64)
+                degrid_wave_kernel<MODE, PATH><<<g, b, 0, st>>>(d);
+        } else if (lane) {
+            switch (d.g.W) {
+                case 3: degrid_aa_kernel<MODE, PATH, 3><<<g, b, smem, st>>>(d); break;
+                case 5: degrid_aa_kernel<MODE, PATH, 5><<<g, b, smem, st>>>(d); break;
+                case 7: degrid_aa_kernel<MODE, PATH, 7><<<g, b, smem, st>>>(d); break;
+                case 9: degrid_aa_kernel<MODE, PATH, 9><<<g, b, smem, st>>>(d); break;
+                case 11: degrid_aa_kernel<MODE, PATH, 11><<<g, b, smem, st>>>(d); break;
+            }
+        } else if (d.wproj) {
+            degrid_group_kernel<MODE, PATH, true><<<g, b, 0, st>>>(d);
+        } else {
+            degrid_group_kernel<MODE, PATH, false><<<g, b, 0, st>>>(d);
         }
-    return hipGetLastError();
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <int MODE> static hipError_t launch_m(const DArgs &d, int path, hipStream_t st) {
