@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/bullseye_amd.h"
+#include "sincos_unit.h"
 
 namespace bam {
 
@@ -143,30 +144,6 @@ template <typename T> __device__ __forceinline__ cpx<T> cmac(cpx<T> acc, cpx<T> 
 template <typename T>
 __device__ __forceinline__ cpx<T> cmac_conj(cpx<T> acc, cpx<T> a, cpx<T> b) {
     return {fma(a.re, b.re, fma(a.im, b.im, acc.re)), fma(a.im, b.re, fma(-a.re, b.im, acc.im))};
-}
-
-// sin and cos of pi x for |x| <= 1, FP32: x = n/2 + r exactly, |r| <= 1/4, and polynomials in
-// r^2 fitted by Remez exchange (the sine's constant term is pi minus its FP32 value, so the
-// leading product carries pi to 48 bits).  Below 0.97 ulp everywhere (3.1 M arguments against
-// extended precision); about 24 instructions, where sincospif spends 45 on arguments it has to
-// reduce and classify first.
-__device__ __forceinline__ void sincospi_unit(float x, float *sn, float *cs) {
-    const float n = rintf(2.0f * x);
-    const float r = fmaf(n, -0.5f, x);
-    const float z = r * r;
-    float u = fmaf(z, 0x1.4bc89ap-4f, -0x1.32ca9ep-1f);
-    u = fmaf(u, z, 0x1.466bbap+1f);
-    u = fmaf(u, z, -0x1.4abbcep+2f);
-    u = fmaf(u, z, -0x1.778948p-24f);
-    const float s = fmaf(0x1.921fb6p+1f, r, r * u);
-    float v = fmaf(z, 0x1.d9f7bcp-3f, -0x1.55c664p+0f);
-    v = fmaf(v, z, 0x1.03c1dep+2f);
-    v = fmaf(v, z, -0x1.3bd3ccp+2f);
-    const float c = fmaf(v, z, 1.0f);
-    const uint32_t q = (uint32_t)(int)n;
-    const uint32_t a = __float_as_uint((q & 1u) ? c : s), b = __float_as_uint((q & 1u) ? s : c);
-    *sn = __uint_as_float(a ^ ((q & 2u) << 30));
-    *cs = __uint_as_float(b ^ (((q + 1u) & 2u) << 30));
 }
 
 // Kahan-compensated running sum of one real component.  The true sum is s - c.
