@@ -173,25 +173,30 @@ hipError_t abi_to_grid(const void *in, double *g, uint64_t slices_fc, uint32_t P
 // then).
 __global__ void k_fold_slots(double *p, uint64_t stride, uint32_t nslots, double *host,
                              const int *err) {
-    const uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64;
-    if (i >= stride || (err && *err)) return;
+    if (err && *err) return;
     const uint32_t lane = threadIdx.x & 63;
-    double s = 0.0;
-    for (uint32_t j = lane; j < nslots; j += 64) {
-        s += p[(uint64_t)j * stride + i];
-        if (j) p[(uint64_t)j * stride + i] = 0.0;
-    }
-    s = wave_sum(s);
-    if (lane == 0) {
-        p[i] = s;
-        if (host) host[i] = s;
+    for (uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64; i < stride;
+         i += (uint64_t)gridDim.x * blockDim.x / 64) {
+        double s = 0.0;
+        for (uint32_t j = lane; j < nslots; j += 64) {
+            s += p[(uint64_t)j * stride + i];
+            if (j) p[(uint64_t)j * stride + i] = 0.0;
+        }
+        s = wave_sum(s);
+        if (lane == 0) {
+            p[i] = s;
+            if (host) host[i] = s;
+        }
     }
 }
 
 hipError_t fold_slots(double *p, uint64_t stride, uint32_t nslots, hipStream_t st, double *host,
                       const int *err) {
     if (!stride || (nslots < 2 && !host)) return hipSuccess;
-    k_fold_slots<<<nblk(stride * 64), 256, 0, st>>>(p, stride, nslots, host, err);
+    // (a launch holds fewer than 2^32 work items)
+    const uint64_t blocks = (stride + 3) / 4;
+    k_fold_slots<<<(unsigned)(blocks < 65536 ? blocks : 65536), 256, 0, st>>>(p, stride, nslots,
+                                                                             host, err);
     return hipGetLastError();
 }
 

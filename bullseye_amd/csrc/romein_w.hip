@@ -415,6 +415,7 @@ template <int MODE, int PATH, int W> struct GridderW {
         const int gl = lane - gw * G;
         if (gw >= GPW) return;
         const uint64_t stream =
+            a.first_stream +
             ((uint64_t)xcd_block() * (BLOCK / 64) + (threadIdx.x >> 6)) * (uint64_t)GPW + gw;
         if (stream >= a.n_streams) return;
         uint64_t t = stream;
@@ -741,7 +742,7 @@ template <int MODE, int PATH> struct Wave4 {
                                                 unsigned long long &cnt) {
         const int lane = threadIdx.x & 63;
         const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const uint64_t stream = (uint64_t)xcd_block() * (BLOCK / 64) + wave;
+        const uint64_t stream = a.first_stream + (uint64_t)xcd_block() * (BLOCK / 64) + wave;
         if (stream >= a.n_streams) return;
         uint64_t t = stream;
         const uint32_t facet = (uint32_t)(t % a.facets);
@@ -917,13 +918,10 @@ void romein_w_kernel(GridArgs a) {
     }
 }
 
-template <int MODE, int PATH, int W> static hipError_t launch_t(const GridArgs &a, hipStream_t st) {
+template <int MODE, int PATH, int W> static hipError_t launch_t(GridArgs a, hipStream_t st) {
     typedef GridderW<MODE, PATH, W> Gd;
     constexpr bool one = one_per_wave(MODE, PATH, W);
     constexpr int gpw = one ? 1 : Gd::GPW;
-    const uint64_t waves = (a.n_streams + gpw - 1) / gpw;
-    const uint64_t blocks = (waves + BLOCK / 64 - 1) / (BLOCK / 64);
-    if (blocks == 0) return hipSuccess;
     size_t wave_bytes = Gd::WAVE_BYTES;
     if constexpr (one) wave_bytes = Wave4<MODE, PATH>::WAVE_BYTES;
     const size_t smem = ((rot_table_len(a.OS, W) * sizeof(typename Gd::T) + 15) & ~15u) +
@@ -931,8 +929,16 @@ template <int MODE, int PATH, int W> static hipError_t launch_t(const GridArgs &
                         (((size_t)a.spw_count * a.chan * sizeof(ChanRec) + 15) & ~(size_t)15) +
                         (BLOCK / 64) * wave_bytes;
     if (!a.rowrec || !a.chanrec) return hipErrorInvalidValue;
-    romein_w_kernel<MODE, PATH, W><<<dim3((uint32_t)blocks), dim3(BLOCK), smem, st>>>(a);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 work items, 67 M streams of one wavefront each
+    constexpr uint64_t per_block = (uint64_t)gpw * (BLOCK / 64), piece = per_block << 23;
+    for (a.first_stream = 0; a.first_stream < a.n_streams; a.first_stream += piece) {
+        const uint64_t left = a.n_streams - a.first_stream;
+        const uint64_t blocks = ((left < piece ? left : piece) + per_block - 1) / per_block;
+        romein_w_kernel<MODE, PATH, W><<<dim3((uint32_t)blocks), dim3(BLOCK), smem, st>>>(a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <int MODE, int W> static hipError_t launch_p(const GridArgs &a, int path, hipStream_t st) {
