@@ -56,6 +56,14 @@ __device__ __forceinline__ int mod_m(int v, int M) {
     return v >= M ? v - M : v;
 }
 
+// Plane of channel c at |w| metres, operation by operation as the gridders form it (w times the
+// rounded reciprocal of the wavelength): a quotient can fall on the other side of a plane boundary.
+__device__ __forceinline__ double stream_plane(const GridArgs &a, double w, uint32_t spw,
+                                               uint32_t c, uint32_t wplanes, float wmax_f) {
+    const double rw = 1.0 / (double)a.wavelengths[spw * a.chan + c];
+    return rint(w * rw / (double)wmax_f * (double)(wplanes - 1));
+}
+
 // Support class of every stream: the widest plane (2 S_p + 1) any of its samples can use.
 __global__ void k_stream_class(GridArgs a, const uint32_t *plane_half, uint32_t wplanes,
                                float wmax_f, uint32_t nseg_max, uint32_t seg_rows, uint8_t *cls) {
@@ -76,8 +84,7 @@ __global__ void k_stream_class(GridArgs a, const uint32_t *plane_half, uint32_t 
         if (spw >= a.spw_count) continue;
         const double w = fabs((double)a.uvw[3 * (size_t)row + 2]);
         for (uint32_t c = c_lo; c < c_hi; ++c) {
-            const double wl = w / (double)a.wavelengths[spw * a.chan + c];
-            const double pl = rint(wl / (double)wmax_f * (double)(wplanes - 1));
+            const double pl = stream_plane(a, w, spw, c, wplanes, wmax_f);
             if (pl < (double)wplanes) best = max(best, (int)(2 * plane_half[(int)pl] + 1));
         }
     }
@@ -1336,8 +1343,7 @@ __global__ void k_entry_class(GridArgs a, const uint32_t *seg_first, const uint3
             if (spw >= a.spw_count) continue;
             const double w = fabs((double)a.uvw[3 * (size_t)row + 2]);
             for (uint32_t c = c_lo; c < c_hi; ++c) {
-                const double wl = w / (double)a.wavelengths[spw * a.chan + c];
-                const double pl = rint(wl / (double)wmax_f * (double)(wplanes - 1));
+                const double pl = stream_plane(a, w, spw, c, wplanes, wmax_f);
                 if (pl < (double)wplanes) best = max(best, (int)(2 * plane_half[(int)pl] + 1));
             }
         }
