@@ -512,7 +512,8 @@ int capture(Plan &pl, hipStream_t st) {
 }
 
 // The passes of the tiled gridder: facets of one kind together while their samples' records stay
-// within 4 GiB (halved while the workspace cannot be had), rows split where one facet's do not.
+// within 4 GiB (halved while the workspace cannot be had) or the options' records per pass, rows
+// split where one facet's do not.
 // pl.tiled stays false where a facet's bins cannot be numbered.
 int plan_tiles(Plan &pl) {
     const LibView lv = lib_view();
@@ -537,7 +538,8 @@ int plan_tiles(Plan &pl) {
         size_t ws = 0;
         for (int kind : {pl.mode, (int)MODE_PSF}) {
             const uint32_t nc = kind == MODE_PSF ? 1 : pl.NC;
-            const uint64_t cap = bytes / (sizeof(wt::Head) + 4 + (size_t)nc * (fp64 ? 16 : 8));
+            uint64_t cap = bytes / (sizeof(wt::Head) + 4 + (size_t)nc * (fp64 ? 16 : 8));
+            if (lv.tile_records) cap = std::min(cap, lv.tile_records);
             const uint64_t rows1 = std::max<uint64_t>(
                 1, std::min<uint64_t>(pl.rows, cap / std::max<uint64_t>(1, per_row)));
             const uint64_t samples1 = std::max<uint64_t>(1, rows1 * per_row);

@@ -109,6 +109,7 @@ struct LibView {
     bool device_resident;
     int path;            // resolved compute path
     int walk_order;      // bullseye_options::walk_order
+    uint64_t tile_records;   // bullseye_options::reserved[1]
     int *errflag;        // device error bits
     unsigned long long *counters;  // device [nslots][2] samples, taps
     uint32_t nslots;

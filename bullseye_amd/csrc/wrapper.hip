@@ -872,6 +872,7 @@ LibView lib_view() {
     v.device_resident = g.opts.device_resident != 0;
     v.path = g.path;
     v.walk_order = (int)g.opts.walk_order;
+    v.tile_records = g.opts.reserved[1];
     v.errflag = g.errflag.as<int>();
     v.counters = g.counters.as<unsigned long long>();
     v.nslots = g.nslots;

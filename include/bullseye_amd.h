@@ -207,7 +207,8 @@ typedef struct bullseye_options {
                                    channels inner; 2 = time inner */
     uint32_t reserved[9];       /* reserved[0]: bit 0 forces the generic (any-support) AA
                                    kernel, bit 1 the w-projection class kernels; reserved[1]:
-                                   w-projection records per pass (0 = up to 4 GiB of them) */
+                                   w-projection records per pass of a call or a batch (0 = up
+                                   to 4 GiB of them) */
 } bullseye_options;
 
 int bullseye_set_options(const bullseye_options *options);
