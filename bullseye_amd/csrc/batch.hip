@@ -514,7 +514,8 @@ int capture(Plan &pl, hipStream_t st) {
 // The passes of the tiled gridder: facets of one kind together while their samples' records stay
 // within 4 GiB (halved while the workspace cannot be had) or the options' records per pass, rows
 // split where one facet's do not.
-// pl.tiled stays false where a facet's bins cannot be numbered.
+// pl.tiled stays false where a facet's bins cannot be numbered or the smallest workspace cannot be
+// had: the class lists then take the batch.
 int plan_tiles(Plan &pl) {
     const LibView lv = lib_view();
     const bool fp64 = pl.path == PATH_FP64;
@@ -589,10 +590,13 @@ int plan_tiles(Plan &pl) {
                 }
             }
         }
-        const hipError_t e = pl.tile_ws.ensure(std::max<size_t>(ws, 16));
-        if (e == hipErrorOutOfMemory && bytes > ((uint64_t)16 << 20)) {
-            (void)hipGetLastError();
-            continue;
+        const hipError_t e = ws > lv.tile_bytes ? hipErrorOutOfMemory
+                                                : pl.tile_ws.ensure(std::max<size_t>(ws, 16));
+        if (e == hipErrorOutOfMemory) {
+            if (bytes > ((uint64_t)16 << 20)) continue;
+            pl.tile_ws.release();
+            pl.passes.clear();
+            return 0;
         }
         HIP_TRY(e);
         break;

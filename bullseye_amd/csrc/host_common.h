@@ -82,7 +82,10 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
         hipError_t e = hipMalloc(&p, n ? n : 16);
-        if (e == hipSuccess) bytes = n;
+        if (e == hipSuccess)
+            bytes = n;
+        else
+            (void)hipGetLastError();
         return e;
     }
     void release() {
@@ -110,6 +113,7 @@ struct LibView {
     int path;            // resolved compute path
     int walk_order;      // bullseye_options::walk_order
     uint64_t tile_records;   // bullseye_options::reserved[1]
+    size_t tile_bytes;       // bullseye_options::reserved[2], in bytes (SIZE_MAX: no bound)
     int *errflag;        // device error bits
     unsigned long long *counters;  // device [nslots][2] samples, taps
     uint32_t nslots;

@@ -128,6 +128,11 @@ int fail(const char *fmt, ...) {
 
 static bool dev_mode() { return g.opts.device_resident != 0; }
 
+// Most bytes of a tiled workspace (bullseye_options::reserved[2], MiB).
+static size_t tile_bytes() {
+    return g.opts.reserved[2] ? (size_t)g.opts.reserved[2] << 20 : SIZE_MAX;
+}
+
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Device memory for one of a gridding call's tables: carved from the scratch arena inside
@@ -560,7 +565,9 @@ static int grid_classes(GridArgs a, size_t rows, size_t B, float wmax_f, const v
 }
 
 // W-projection through on-chip tiles (wtile.hip), in passes over facets (and rows, where one
-// facet's samples are too many) whose records fit the workspace.  tiled: whether it applied.
+// facet's samples are too many) whose records fit the workspace.  tiled: whether it applied; not
+// where the bins cannot be numbered or the smallest workspace cannot be had (the counters and
+// items do not shrink with the records).
 static int grid_tiles(const GridArgs &a, size_t rows, float wmax_f, const void *taps, int mode,
                       bool &tiled) {
     tiled = !(g.opts.reserved[0] & 2);
@@ -576,23 +583,36 @@ static int grid_tiles(const GridArgs &a, size_t rows, float wmax_f, const void *
     }
     const uint64_t spots1 = (uint64_t)a.cube * wt::tiles_of(a.nx) * wt::tiles_of(a.ny);
     const size_t rec = sizeof(wt::Head) + 4 + (size_t)nc * (fp64 ? 16 : 8);
+    if (g.wtile.bytes > tile_bytes()) g.wtile.release();   // (hipFree waits for what uses it)
     // 4 GiB of records, halved while the workspace cannot be had
     for (uint64_t cap = g.opts.reserved[1] ? g.opts.reserved[1] : ((size_t)4 << 30) / rec;;
          cap /= 2) {
         const uint64_t rows1 = std::min<uint64_t>(rows, std::max<uint64_t>(1, cap / a.chan));
         uint64_t F1 = std::max<uint64_t>(1, cap / (rows * a.chan));
         F1 = std::min<uint64_t>(std::min<uint64_t>(F1, a.facets), 65535);
-        wt::Plan pl;
-        while (F1 > 1 && !wtile_plan(pl, rows1 * a.chan * F1, spots1 * F1, lo, hi, nc, fp64))
-            F1 = (F1 + 1) / 2;
-        if (!wtile_plan(pl, rows1 * a.chan * F1, spots1 * F1, lo, hi, nc, fp64)) {
+        auto plan = [&](wt::Plan &pl, uint64_t nf, uint64_t nr) {
+            const uint64_t samples = nr * a.chan * nf, spots = spots1 * nf;
+            return (pl.total && pl.samples == samples && pl.spots == spots) ||
+                   wtile_plan(pl, samples, spots, lo, hi, nc, fp64);
+        };
+        wt::Plan pl{};
+        while (F1 > 1 && !plan(pl, F1, rows1)) F1 = (F1 + 1) / 2;
+        // the last pass over the facets or rows may hold fewer; its bins are planned for itself
+        size_t bytes = 0;
+        for (uint64_t nf : {F1, (a.facets - 1) % F1 + 1})
+            for (uint64_t nr : {rows1, (rows - 1) % rows1 + 1}) {
+                if (!plan(pl, nf, nr)) {
+                    tiled = false;
+                    return 0;
+                }
+                bytes = std::max(bytes, pl.total);
+            }
+        const hipError_t e = bytes > tile_bytes() ? hipErrorOutOfMemory : g.wtile.ensure(bytes);
+        if (e == hipErrorOutOfMemory) {
+            if (cap > (1u << 20)) continue;
+            g.wtile.release();
             tiled = false;
             return 0;
-        }
-        const hipError_t e = g.wtile.ensure(pl.total);
-        if (e == hipErrorOutOfMemory && cap > (1u << 20)) {
-            (void)hipGetLastError();
-            continue;
         }
         HIP_TRY(e);
         wt::TArgs t{};
@@ -612,13 +632,9 @@ static int grid_tiles(const GridArgs &a, size_t rows, float wmax_f, const void *
                 t.nfacets = (uint32_t)std::min<uint64_t>(F1, a.facets - f0);
                 t.row0 = (uint32_t)r0;
                 t.row1 = (uint32_t)std::min<uint64_t>(rows, r0 + rows1);
-                // the last pass may hold fewer facets or rows: its bins are planned for itself
-                wt::Plan one;
-                if (!wtile_plan(one, (uint64_t)(t.row1 - t.row0) * a.chan * t.nfacets,
-                                spots1 * t.nfacets, lo, hi, nc, fp64))
+                if (!plan(pl, t.nfacets, t.row1 - t.row0))
                     return fail("w-projection workspace plan");
-                HIP_TRY(g.wtile.ensure(one.total));
-                HIP_TRY(wtile_grid(t, one, g.wtile.p, mode, fp64, widths, g.stream, g.wside,
+                HIP_TRY(wtile_grid(t, pl, g.wtile.p, mode, fp64, widths, g.stream, g.wside,
                                    State::WSIDE, g.wfork, g.wjoin));
             }
         return 0;
@@ -873,6 +889,7 @@ LibView lib_view() {
     v.path = g.path;
     v.walk_order = (int)g.opts.walk_order;
     v.tile_records = g.opts.reserved[1];
+    v.tile_bytes = tile_bytes();
     v.errflag = g.errflag.as<int>();
     v.counters = g.counters.as<unsigned long long>();
     v.nslots = g.nslots;

@@ -7,7 +7,9 @@ namespace wt {
 
 constexpr int TILE = 33;          // footprint origins per tile and axis (32 + 1: see the bank layout)
 constexpr uint32_t COPIES = 16;   // counters per bin (at most), so a busy bin's atomics spread
-constexpr uint64_t MAX_SLOTS = 1ull << 27;   // counters of one pass (0.5 GiB)
+// Counters of one pass at most.  The workspace beside the records is then 0.5 GiB of counters, as
+// much of first places, and up to 3 GiB of work items.
+constexpr uint64_t MAX_SLOTS = 1ull << 27;
 
 __host__ __device__ constexpr uint32_t tiles_of(uint32_t n) { return (n + TILE - 1) / TILE; }
 

@@ -208,7 +208,10 @@ typedef struct bullseye_options {
     uint32_t reserved[9];       /* reserved[0]: bit 0 forces the generic (any-support) AA
                                    kernel, bit 1 the w-projection class kernels; reserved[1]:
                                    w-projection records per pass of a call or a batch (0 = up
-                                   to 4 GiB of them) */
+                                   to 4 GiB of them); reserved[2]: most MiB of workspace that the
+                                   tiled w-projection takes for the calls together or for a
+                                   batch plan (0 = what can be had; the records are halved until
+                                   they fit, then the class kernels run) */
 } bullseye_options;
 
 int bullseye_set_options(const bullseye_options *options);
