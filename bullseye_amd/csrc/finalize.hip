@@ -356,8 +356,8 @@ static hipError_t fft_plan(uint32_t nx, uint32_t ny, uint32_t batch, hipfftHandl
     FftPlan p = {nullptr, nx, ny, batch};
     if (hipfftPlanMany(&p.h, 2, dims, nullptr, 1, npix, nullptr, 1, npix, type, (int)batch) !=
         HIPFFT_SUCCESS) {
-        // the kept plans' work areas may be what is missing
-        finalize_release_plans();
+        // what is kept for later calls, other plans' work areas too, may be what is missing
+        release_idle_memory();
         if (hipfftPlanMany(&p.h, 2, dims, nullptr, 1, npix, nullptr, 1, npix, type, (int)batch) !=
             HIPFFT_SUCCESS)
             return hipErrorUnknown;

@@ -73,6 +73,12 @@ hipError_t launch_facet_geom(const uvw_base_type *fc, double ra0, double dec0, u
 // cpu_gpu_common/cu_common.h:63 -- a float constant in every precision build
 static const float ARCSEC_TO_RAD = (float)(M_PI / (180.0 * 3600.0));
 
+// Gives back the memory that the context keeps between calls and can do without: the single calls'
+// tiled workspace and the FFT plans.  Waits for the stream.
+void release_idle_memory();
+
+// A device buffer that grows.  Where the memory is short, what the context keeps for later calls
+// goes first; a failure is the caller's to report and not the next launch's.
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
@@ -82,6 +88,11 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
         hipError_t e = hipMalloc(&p, n ? n : 16);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            release_idle_memory();
+            e = hipMalloc(&p, n ? n : 16);
+        }
         if (e == hipSuccess)
             bytes = n;
         else

@@ -133,6 +133,12 @@ static size_t tile_bytes() {
     return g.opts.reserved[2] ? (size_t)g.opts.reserved[2] << 20 : SIZE_MAX;
 }
 
+void release_idle_memory() {
+    if (g.stream) (void)hipStreamSynchronize(g.stream);
+    g.wtile.release();
+    finalize_release_plans();
+}
+
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Device memory for one of a gridding call's tables: carved from the scratch arena inside

@@ -1,5 +1,6 @@
 """Device memory of the tiled w-projection gridder: a call or a batch plan that the allowed (or
-available) workspace cannot hold runs on the class kernels.
+available) workspace cannot hold runs on the class kernels, and what the context keeps between
+calls is given back when another allocation needs it.
 
 A 4096^2 grid of 32 widths takes 15625 tiles x 32 x 16 counters of 4 bytes, and as many first places:
 64 MB whatever the records.  Bars between the two kernels as in test_gpu_wproj for FP64."""
@@ -94,3 +95,34 @@ def test_batch_beyond_the_workspace(context):
         batch.kernel_set(0, context.spec.conv, 31, 1, context.halves, context.spec.wmax)
     assert held[1] - held[0] >= FIXED - 32 * MB   # the class kernels' lists take some too
     close(got[0], got[1])
+
+
+def test_kept_memory_is_given_back(context):
+    print("case workspace given back", flush=True)
+    context.grid(mib=16)
+    held = free_bytes()
+    want = context.grid()
+    assert held - free_bytes() >= FIXED
+    # a plan whose grids exceed any GPU (20 of 45000^2 cells of 16 bytes: 648 GB) is refused, and
+    # asking for them has taken what the calls keep
+    batch = FacetBatch(context.lib, context.b)
+    batch.kernel_set(0, context.spec.conv, 31, 1, context.halves, context.spec.wmax)
+    table = [BatchFacet(45000, context.spec.cell, context.obs.phase_centre, 0)] * 20
+    refuse(batch, table)
+    batch.release()
+    assert held - free_bytes() <= 8 * MB
+    close(context.grid(), want)
+
+
+def refuse(batch, facets):
+    """bullseye_batch_plan without the facets' outputs."""
+    from bullseye_amd.batch import GRID_MODES
+    from bullseye_amd.library_loader import bullseye_batch_facet
+    table = (bullseye_batch_facet * len(facets))()
+    for e, f in zip(table, facets):
+        e.nx = e.ny = f.npix
+        e.kernel_set, e.cell_x, e.cell_y = f.kernel_set, f.cell, f.cell
+        e.ra, e.dec = f.centre
+    assert batch.lib.bullseye_batch_plan(batch.binding.byref(), GRID_MODES[batch.mode], table,
+                                         len(facets), 0) != 0
+    assert b"memory" in batch.lib.bullseye_last_error(), batch.lib.bullseye_last_error()
