@@ -759,7 +759,7 @@ static int grid_call(gridding_parameters *p, int mode, bool facet, bool phase,
         if (!tiled && grid_classes(a, rows, B, wmax_f, taps, mode)) return 1;
     } else {
         const bool specialised = romein_w_groups_per_wave(W, mode, g.path) > 0 &&
-                                 !(g.opts.reserved[0] & 1);
+                                 !g.opts.reserved[0];
         if (specialised) {
             const bool four = mode == MODE_4 || mode == MODE_4J;
             a.pol_contig = (four && !psf && p->number_of_polarization_terms == 4 &&

@@ -205,8 +205,9 @@ typedef struct bullseye_options {
     uint32_t walk_order;        /* order of a stream's samples: 0 = whichever moves the kernel
                                    footprint less per step, measured from the data; 1 =
                                    channels inner; 2 = time inner */
-    uint32_t reserved[9];       /* reserved[0]: bit 0 forces the generic (any-support) AA
-                                   kernel, bit 1 the w-projection class kernels; reserved[1]:
+    uint32_t reserved[9];       /* reserved[0]: any nonzero value forces the generic
+                                   (any-support) AA kernel, bit 1 the w-projection class kernels
+                                   as well; reserved[1]:
                                    w-projection records per pass of a call or a batch (0 = up
                                    to 4 GiB of them); reserved[2]: most MiB of workspace that the
                                    tiled w-projection takes for the calls together or for a
