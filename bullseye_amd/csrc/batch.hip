@@ -880,7 +880,8 @@ bool default_tiles(const bullseye_batch_tuning &t) {
 int plan_impl(gridding_parameters *p, int mode, const bullseye_batch_facet *facets, uint32_t n,
               int schedule) {
     if (build_plan(p, mode, facets, n, schedule, tuning, plan,
-                   schedule != BULLSEYE_BATCH_PER_FACET && default_tiles(tuning)))
+                   schedule != BULLSEYE_BATCH_PER_FACET && default_tiles(tuning) &&
+                       !lib_view().wproj_classes))
         return 1;
     if (schedule == BULLSEYE_BATCH_PERSISTENT_GRAPH && capture(plan, lib_view().stream)) return 1;
     plan.ready = true;
@@ -1084,7 +1085,7 @@ int autotune_impl(gridding_parameters *p, int mode, const bullseye_batch_facet *
     best_t.facet_major = order_ms[1] < order_ms[0] ? 1 : 0;
     best_total = std::min(order_ms[0], order_ms[1]);
     // the tiled gridder, which the default tiles stand for, against the tuned class kernels
-    {
+    if (!lv.wproj_classes) {
         bullseye_batch_tuning t = best_t;
         for (uint32_t i = 0; i < NCLS; ++i) t.shape[i] = t.chunk[i] = 0;
         t.facet_major = 0;

@@ -123,6 +123,7 @@ struct LibView {
     bool device_resident;
     int path;            // resolved compute path
     int walk_order;      // bullseye_options::walk_order
+    bool wproj_classes;      // bullseye_options::reserved[0], bit 1
     uint64_t tile_records;   // bullseye_options::reserved[1]
     size_t tile_bytes;       // bullseye_options::reserved[2], in bytes (SIZE_MAX: no bound)
     int *errflag;        // device error bits

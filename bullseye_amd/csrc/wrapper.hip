@@ -894,6 +894,7 @@ LibView lib_view() {
     v.device_resident = g.opts.device_resident != 0;
     v.path = g.path;
     v.walk_order = (int)g.opts.walk_order;
+    v.wproj_classes = (g.opts.reserved[0] & 2) != 0;
     v.tile_records = g.opts.reserved[1];
     v.tile_bytes = tile_bytes();
     v.errflag = g.errflag.as<int>();

@@ -207,7 +207,7 @@ typedef struct bullseye_options {
                                    channels inner; 2 = time inner */
     uint32_t reserved[9];       /* reserved[0]: any nonzero value forces the generic
                                    (any-support) AA kernel, bit 1 the w-projection class kernels
-                                   as well; reserved[1]:
+                                   as well (in calls, batch plans and the autotuner); reserved[1]:
                                    w-projection records per pass of a call or a batch (0 = up
                                    to 4 GiB of them); reserved[2]: most MiB of workspace that the
                                    tiled w-projection takes for the calls together or for a
@@ -365,7 +365,8 @@ enum bullseye_batch_schedule {
  * lane) and chunk[i] the classification segments per work item (1, 2 or 4: the visibility
  * chunk length is chunk * base_rows rows).  channels_per_stream and base_rows are shared by all
  * classes (0: automatic, 32).  With every shape at 0, every chunk at most 1 and facet_major 0 the
- * facets run through on-chip tiles instead of the class kernels these choices are for. */
+ * facets run through on-chip tiles instead of the class kernels these choices are for, unless the
+ * options force the class kernels. */
 typedef struct bullseye_batch_tuning {
     uint32_t struct_size;       /* sizeof(bullseye_batch_tuning) */
     uint32_t channels_per_stream;
@@ -378,7 +379,9 @@ typedef struct bullseye_batch_tuning {
                                    together (its grid's atomics local in the memory-side cache) */
     uint32_t reserved;
     double tuned_ms;            /* autotune: summed device time of the chosen launches */
-    double default_ms;          /* autotune: the same with the default tiles */
+    double default_ms;          /* autotune: the same with the default tiles: a pass through
+                                   the on-chip tiles, or, where the options force them, the
+                                   class kernels' default launches */
 } bullseye_batch_tuning;
 int bullseye_batch_set_tuning(const bullseye_batch_tuning *tuning);
 int bullseye_batch_get_tuning(bullseye_batch_tuning *tuning);
