@@ -15,12 +15,17 @@ namespace bam {
 
 typedef visibility_base_type vis_t;
 
+// The element of this lane in a launch of nblk(n) blocks.
+__device__ __forceinline__ uint64_t element() {
+    return ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+}
+
 // internal FP64 accumulation grid [F][C][ny][nx][pstride][2] <-> ABI grid
 // complex<grid_base_type>[F][C][P][ny][nx]
 // (err: nothing is written while the device error flag is set)
 __global__ void k_grid_to_abi(const double *g, grid_base_type *out, uint64_t slices_fc, uint32_t P,
                               uint32_t pstride, uint64_t npix, const int *err) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     const uint64_t total = slices_fc * npix;
     if (i >= total || (err && *err)) return;
     const uint64_t fc = i / npix, pix = i - fc * npix;
@@ -34,7 +39,7 @@ __global__ void k_grid_to_abi(const double *g, grid_base_type *out, uint64_t sli
 
 __global__ void k_abi_to_grid(const grid_base_type *in, double *g, uint64_t slices_fc, uint32_t P,
                               uint32_t pstride, uint64_t npix) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     const uint64_t total = slices_fc * npix;
     if (i >= total) return;
     const uint64_t fc = i / npix, pix = i - fc * npix;
@@ -52,13 +57,13 @@ __global__ void k_abi_to_grid(const grid_base_type *in, double *g, uint64_t slic
 }
 
 __global__ void k_fill_f64(double *p, uint64_t n, double v) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     if (i < n) p[i] = v;
 }
 
 // cpu_algorithm/wrapper.cpp:136-163: slice (f, ch, corr) /= (grid type)norm[(f*C+ch)*P+corr]
 __global__ void k_normalize(grid_base_type *out, const double *norm, uint64_t slices, uint64_t npix) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     if (i >= slices * npix) return;
     const grid_base_type d = (grid_base_type)norm[i / npix];
     out[2 * i] /= d;
@@ -70,7 +75,7 @@ __global__ void k_normalize(grid_base_type *out, const double *norm, uint64_t sl
 __global__ void k_weight_uniformly(grid_base_type *out, const grid_base_type *sf,
                                    const uint64_t *cgi, uint32_t F, uint32_t C, uint32_t P,
                                    uint32_t sfC, uint64_t npix) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     if (i >= (uint64_t)F * C * npix) return;
     const uint64_t fg = i / npix, pix = i - fg * npix;
     const uint64_t f = fg / C, g = fg - f * C;
@@ -90,7 +95,7 @@ __global__ void k_weight_uniformly(grid_base_type *out, const grid_base_type *sf
 __global__ void k_ifftshift_gather(const grid_base_type *in, grid_base_type *out, uint32_t F,
                                    uint32_t n, uint32_t fstride, uint32_t nx, uint32_t ny) {
     const uint64_t npix = (uint64_t)nx * ny;
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     if (i >= (uint64_t)F * n * npix) return;
     const uint64_t s = i / npix, pix = i - s * npix;
     const uint32_t f = (uint32_t)(s / n), k = (uint32_t)(s - (uint64_t)f * n);
@@ -111,7 +116,7 @@ __global__ void k_fftshift_scatter(const grid_base_type *in, grid_base_type *out
                                    uint32_t n, uint32_t fstride, uint32_t nx, uint32_t ny,
                                    const double *tx, const double *ty, int reals) {
     const uint64_t npix = (uint64_t)nx * ny;
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     if (i >= (uint64_t)F * n * npix) return;
     const uint64_t s = i / npix, pix = i - s * npix;
     const uint32_t f = (uint32_t)(s / n), k = (uint32_t)(s - (uint64_t)f * n);
@@ -149,7 +154,14 @@ __global__ void k_fftshift_scatter(const grid_base_type *in, grid_base_type *out
     }
 }
 
-static inline unsigned nblk(uint64_t n) { return (unsigned)((n + 255) / 256); }
+// Blocks of 256 for n elements, in rows: a launch of 2^32 work items along one axis or more is cut
+// short without an error, and grids of 34 GB reach that.
+static inline dim3 nblk(uint64_t n) {
+    constexpr uint64_t ROW = 1u << 20;
+    const uint64_t blocks = (n + 255) / 256;
+    return blocks <= ROW ? dim3((unsigned)blocks)
+                         : dim3((unsigned)ROW, (unsigned)((blocks + ROW - 1) / ROW));
+}
 
 hipError_t grid_to_abi(const double *g, void *out, uint64_t slices_fc, uint32_t P,
                        uint32_t pstride, uint64_t npix, hipStream_t st, const int *err) {
@@ -239,7 +251,7 @@ hipError_t fill_f64(double *p, uint64_t n, double v, hipStream_t st) {
 __global__ void k_stokes_combine(const grid_base_type *g, grid_base_type *tmp, uint32_t F,
                                  uint32_t C, uint32_t P, uint64_t npix, int first, int second,
                                  int sign) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     if (i >= (uint64_t)F * C * npix) return;
     const uint64_t fc = i / npix, px = i - fc * npix;
     const grid_base_type *base = g + 2 * (fc * P * npix + px);
@@ -267,7 +279,7 @@ __global__ void k_stokes_combine(const grid_base_type *g, grid_base_type *tmp, u
 __global__ void k_stokes_place(grid_base_type *g, const grid_base_type *tmp, uint32_t F,
                                uint32_t C, uint32_t P, uint64_t npix, int compact,
                                int contiguous) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = element();
     const uint64_t slots = (uint64_t)C * P;
     if (i >= (uint64_t)F * slots * npix) return;
     const uint64_t fs = i / npix, px = i - fs * npix;
