@@ -114,7 +114,7 @@ struct GridArgs {
     uint32_t pol_idx[4];
     uint32_t imaging_field;
     uint32_t baselines, chan_per_stream, n_chan_blocks, n_segments;
-    uint64_t n_streams, first_stream;   // first_stream: of this launch (romein_w.hip)
+    uint64_t n_streams, first_stream;   // first_stream: of this launch (AA gridders)
     uint64_t norm_stride;                      // facet*cube*ncorr (elements of one slot)
     uint32_t nslots;                           // copies of norm and counters (>= 1)
     double u_scale, v_scale, off_x, off_y;

@@ -222,6 +222,7 @@ template <int MODE, int PATH, bool WPROJ> struct Gridder {
         const int gl = lane - gw * G;
         if (gw >= gpw) return;
         const uint64_t stream =
+            a.first_stream +
             ((uint64_t)xcd_block() * (BLOCK / 64) + wave) * (uint64_t)gpw + (uint64_t)gw;
         if (stream >= a.n_streams) return;
         // stream -> (baseline, channel block, segment, facet); facet fastest so that the
@@ -360,16 +361,20 @@ template <int MODE, int PATH> static size_t smem_bytes(const GridArgs &a) {
 }
 
 template <int MODE, int PATH>
-static hipError_t launch_t(const GridArgs &a, hipStream_t st) {
+static hipError_t launch_t(GridArgs a, hipStream_t st) {
     const int W = (int)a.W;
     const int G = W * ((W + R - 1) / R);
-    const int gpw = 64 / G;
-    const uint64_t waves = (a.n_streams + gpw - 1) / gpw;
-    const uint64_t blocks = (waves + BLOCK / 64 - 1) / (BLOCK / 64);
-    if (blocks == 0) return hipSuccess;
     const size_t smem = smem_bytes<MODE, PATH>(a);
-    romein_aa_kernel<MODE, PATH><<<dim3((uint32_t)blocks), dim3(BLOCK), smem, st>>>(a);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 work items
+    const uint64_t per_block = (uint64_t)(64 / G) * (BLOCK / 64), piece = per_block << 23;
+    for (a.first_stream = 0; a.first_stream < a.n_streams; a.first_stream += piece) {
+        const uint64_t left = a.n_streams - a.first_stream;
+        const uint64_t blocks = ((left < piece ? left : piece) + per_block - 1) / per_block;
+        romein_aa_kernel<MODE, PATH><<<dim3((uint32_t)blocks), dim3(BLOCK), smem, st>>>(a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <int MODE> static hipError_t launch_m(const GridArgs &a, int path, hipStream_t st) {

@@ -1,4 +1,4 @@
-"""AA gridding calls of more streams than one launch of the specialised kernels holds (fewer than
+"""AA gridding calls of more streams than one launch of the gridding kernels holds (fewer than
 2^32 work items, one wavefront a stream for four correlations at W = 7): many baselines and
 facets, few of them with samples, against the oracle.  Bars as in test_gpu_parity for the
 compensated FP32 path."""
@@ -15,9 +15,11 @@ pytestmark = pytest.mark.gpu
 ANTENNAS = 2000   # 2.0 M baselines
 
 
-@pytest.mark.parametrize("mode,facets", [("facet_4_cor", 40), ("facet_duel_pol", 150)])
-def test_many_streams(mode, facets):
-    print("case many streams", mode, facets, flush=True)
+@pytest.mark.parametrize("mode,facets,support", [
+    ("facet_4_cor", 40, 3), ("facet_duel_pol", 150, 3),
+    ("facet_single_pol", 80, 7)])   # W = 15: the generic kernel
+def test_many_streams(mode, facets, support):
+    print("case many streams", mode, facets, support, flush=True)
     obs = round_to(small_obs(mode, n_ant=6, n_time=4, n_chan=3), "mixed")
     # the tracks of the last six antennas: the last streams hold samples too
     obs.ant1 = obs.ant1 + np.uint32(ANTENNAS - 6)
@@ -25,7 +27,7 @@ def test_many_streams(mode, facets):
     obs.ant1[::3] -= np.uint32(ANTENNAS - 6)
     obs.ant2[::3] -= np.uint32(ANTENNAS - 6)
     obs.n_ant = ANTENNAS
-    spec = make_spec(obs, mode, precision="mixed", npix=64, n_facets=facets)
+    spec = make_spec(obs, mode, precision="mixed", npix=64, n_facets=facets, support=support)
     ref = Binding("double", obs, spec)
     oracle.run(ref, mode)
     lib = load_library("GPU", "mixed")
