@@ -432,6 +432,7 @@ def main():
             "ms_per_step": r["ms_per_step"], "fp64_gtaps_per_s": r["fp64_gtaps_per_s"],
             "fp32comp_over_fp64": r["fp32comp_over_fp64"],
             "per_facet_launch_gtaps_per_s": r["per_facet_launch_gtaps_per_s"],
+            "class_kernels_gtaps_per_s": r["class_kernels_gtaps_per_s"],
             "batched_over_per_facet": r["batched_over_per_facet"],
             "rms_err_vs_fp64_gpu_worst_facet": r["rms_err_vs_fp64_gpu_worst_facet"],
             "peak_err_vs_fp64_gpu_worst_facet": r["peak_err_vs_fp64_gpu_worst_facet"],
@@ -818,9 +819,10 @@ def batch_workload(args, steps, warmup, compare_fp64, compare_tiles, cpu):
         if rc != 0:
             raise RuntimeError("%s: %s" % (what, lib.bullseye_last_error().decode()))
 
-    def set_opts(path):
+    def set_opts(path, classes=False):
         o = bullseye_options(struct_size=ctypes.sizeof(bullseye_options), device_resident=1,
                              compute_path=path)
+        o.reserved[0] = 2 if classes else 0   # the w-projection class kernels
         check(lib.bullseye_set_options(ctypes.byref(o)), "options")
 
     spec0 = ImagingSpec(npix=256, cell=im["cell"], conv=kernels.pswf_aa_kernel(3, 63),
@@ -860,8 +862,8 @@ def batch_workload(args, steps, warmup, compare_fp64, compare_tiles, cpu):
             "base rows %d" % (args.tune_timesteps, time.time() - t, tune["tuned_ms"],
                               tune["default_ms"], tune["channels_per_stream"], tune["base_rows"]))
 
-    def run(path, schedule, steps, warmup, what):
-        set_opts(path)
+    def run(path, schedule, steps, warmup, what, classes=False):
+        set_opts(path, classes)
         t = time.time()
         batch.plan(facets, schedule)
         tplan = time.time() - t
@@ -898,15 +900,19 @@ def batch_workload(args, steps, warmup, compare_fp64, compare_tiles, cpu):
             if peak > 0:
                 errs.append((torch.sqrt((d ** 2).mean()).item() / peak, d.max().item() / peak))
         del out32
-        # one launch per (facet, class) of the single-facet kernels, with the tuned tiles
+        # the class kernels with the tuned tiles: all facets in one launch a class, and one launch
+        # per (facet, class)
+        wall_cl, taps_cl, _, _, _ = run(PATH_FP32_KAHAN, BATCH_PERSISTENT_GRAPH, 1, 0,
+                                        "class kernels, persistent graph", classes=True)
         wall_pf, taps_pf, _, _, _ = run(PATH_FP32_KAHAN, BATCH_PER_FACET, 1, 0,
-                                        "one launch per facet and class")
-        assert taps_pf == taps and taps64 == taps
+                                        "class kernels, one launch per facet and class")
+        assert taps_pf == taps and taps64 == taps and taps_cl == taps
         compare = {
             "fp64_gtaps_per_s": round(taps64 / wall64 / 1e9, 3),
             "fp32comp_over_fp64": round(wall64 / wall32, 3),
             "per_facet_launch_gtaps_per_s": round(taps_pf / wall_pf / 1e9, 3),
-            "batched_over_per_facet": round(wall_pf / wall32, 3),
+            "class_kernels_gtaps_per_s": round(taps_cl / wall_cl / 1e9, 3),
+            "batched_over_per_facet": round(wall_pf / wall_cl, 3),   # on the class kernels
             "rms_err_vs_fp64_gpu_worst_facet": max(e[0] for e in errs),
             "peak_err_vs_fp64_gpu_worst_facet": max(e[1] for e in errs)}
         if compare_tiles:
@@ -928,7 +934,8 @@ def batch_workload(args, steps, warmup, compare_fp64, compare_tiles, cpu):
                                "baselines, %d t x 32 ch 1.0-1.5 GHz, 1 corr) into %d facets, "
                                "sizes log-uniform 128^2-2048^2 at 1.5 arcsec, 7 w-kernel stacks "
                                "of 16-128 planes (supports 7->63 by |w|, OS x8), %d sampling-"
-                               "function facets; persistent class launches in one HIP graph"
+                               "function facets; one HIP graph of the on-chip tiles, or of "
+                               "the tuned class kernels where they are faster"
                                % (args.batch_timesteps, nf, n_psf),
                    "rows": obs.rows, "channels": obs.n_chan, "facets": nf,
                    "facet_mpix": round(float((sizes.astype(float) ** 2).sum()) / 1e6, 2),
