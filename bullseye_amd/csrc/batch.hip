@@ -6,8 +6,9 @@
 // visibilities.  Here a plan holds up to 65536 facets over one staged, baseline-sorted
 // visibility set.  At its default tiles the facets of a kind go through the tiled gridder
 // (wtile.hip) in as many passes as their records need (TilePass); 20 facets of 400^2-2048^2 take
-// 4.7 ms there and 9.5 ms on the class kernels' default tiles.  With other tiles, and where a
-// pass cannot number the samples:
+// 4.7 ms there and 9.5 ms on the class kernels' default tiles.  With other tiles, where a
+// pass cannot number the samples or have its workspace, and where the options ask for them, the class
+// kernels:
 //   * every kernel stack ("kernel set") classifies the streams -- (baseline, channel block,
 //     segment of base_rows rows) -- by the widest w-plane any of their samples uses
 //     (k_stream_class, wproj.hip); facets sharing a kernel set share its classes;

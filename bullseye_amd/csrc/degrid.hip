@@ -313,7 +313,7 @@ template <typename T> __device__ __forceinline__ T group_sum(T v) {
 
 // Wavefronts a SIMD the group kernel is scheduled for.  FP64 with Jones terms: scheduled for four
 // (124 registers) its loads wait for each other, 2.06 M samples of a W <= 15 stack take 4.8 ms
-// against 4.2 with three (142 registers).
+// against 3.6 with three (142 registers).
 constexpr int group_waves(int mode, int path) {
     return mode == MODE_4J && path == PATH_FP64 ? 3 : 8;
 }

@@ -74,9 +74,13 @@ template <int MODE, int PATH, int W> struct GridderW {
     typedef Rec<T, NC, W, TR> R_t;
     // Samples of a uniform quad that a compensated run chains (more than a quad: a whole step;
     // otherwise a sample outside uniform quads is a run of its own).  The rounding of a run grows
-    // with its length, so the lengths keep the grids' distance from 64 bits: 2 correlations, W =
-    // 7: 3.3e-8 to 4.2e-8 of the rms (two draws of 1.8 M samples) with runs of a step, 2.7e-8 to
-    // 2.9e-8 with these (rounding the result alone: 2.5e-8).
+    // with its length, so the lengths keep the grids' distance from 64 bits.  FP32 sums in double
+    // grids, rms of six observations of 1.3 M samples, in 1e-8 of the grid's, before the lanes and
+    // registers of 1 and 2 correlations became these and with these lengths:
+    //   W            3           5           7           9           11
+    //   1 corr.  2.35/2.35   2.65/2.65   2.43/2.42   3.17/2.65   3.27/2.88
+    //   2 corr.  2.36/2.36   2.65/2.65   2.43/2.33   3.16/2.65   3.27/2.92
+    // (2 correlations at W = 7 with runs of a step: 20 to 45 % more).
     static constexpr int RUN = NC == 4 ? G + QUAD : NC == 2 && W == 3 ? 1 : NC == 2 && W == 7 ? 2
                                                                                              : QUAD;
     // bytes between the record arrays of consecutive groups: 16-byte aligned and starting

@@ -8,8 +8,9 @@
 // conv[plane][frac_v + j*OS][frac_u + k*OS]; the normalisation adds weight * sum Re(taps).
 //
 // Where these kernels run: most calls and batches go through on-chip tiles (wtile.hip); these class
-// kernels grid the calls whose samples or bins one tiled pass cannot number, the batches whose
-// autotuned tiles are faster, a batch's per-facet schedule, and the calls that ask for them.
+// kernels grid the calls whose samples or bins one tiled pass cannot number or whose workspace
+// cannot be had, the batches whose autotuned tiles are faster, a batch's per-facet schedule, and the
+// calls and batches that ask for them.
 //
 // Variable support.  Each plane p carries its own half support S_p <= S (S = conv_support):
 // its taps outside [S - S_p, S + S_p] are taken as zero (the kernel generator truncates them), so
